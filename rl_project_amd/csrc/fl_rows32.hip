@@ -136,60 +136,31 @@ struct Shared32 {
   uint32_t grp[4];  // next chunk group (wave_groups): two-read path reads 1, 2; top-k path reads 1, 2
 };
 
-// Element source: raw buffer loads of one row (range-checked, so loads past
-// the row return zeros and need no clamping).
+// Element source: 16-byte raw buffer loads of one row.  They need no more than
+// the 4-byte alignment every float row has, and the range check works dword by
+// dword, so a chunk past the row or across its end reads zeros there and needs
+// neither clamping nor a branch.  (Rows of an odd vocabulary, whose starts are
+// not 16-byte aligned, used to go element by element; 30 rows of V = 50257,
+// per launch: top-k 50 16.8 -> 16.2 us, top-p alone 38.0 -> 37.1 us.)
 struct Src {
   __amdgpu_buffer_rsrc_t rs;
   int V;
-  int nfull;  // chunks of 4 elements that lie wholly inside the row
-  bool aligned;
   __device__ __forceinline__ float4 chunk(int c) const {
-    if (aligned && c < nfull) {
-      const uint4 u = buf_load16(rs, 16u * c, 0u);
-      return make_float4(__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w));
-    }
-    float4 f;
-    f.x = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, 16 * c + 0, 0, 0));
-    f.y = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, 16 * c + 4, 0, 0));
-    f.z = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, 16 * c + 8, 0, 0));
-    f.w = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(rs, 16 * c + 12, 0, 0));
-    return f;
+    const uint4 u = buf_load16(rs, 16u * static_cast<uint32_t>(c), 0u);
+    return make_float4(__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w));
   }
-  // chunks c0 + u * NT + tid, u < U.  When all of them are whole chunks of an
-  // aligned row (every iteration of a streaming loop but the last), one
-  // uniform test covers them and each is one 16-byte load; a test per chunk
-  // would put a branch around every load and make the wave wait for all U
-  // loads before it uses the first.  A row of whole chunks (V a multiple of
-  // 4) takes 16-byte loads throughout: a chunk past its end lies wholly
-  // outside the buffer's range and reads zeros.
+  // chunks c0 + u * NT + tid, u < U
   template <int U>
   __device__ __forceinline__ void chunks(int c0, float4 (&q)[U]) const {
-    const int tid = threadIdx.x;
-    if (aligned && (c0 + U * NT <= nfull || 4 * nfull == V)) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const uint4 v = buf_load16(rs, 16u * static_cast<uint32_t>(c0 + u * NT + tid), 0u);
-        q[u] = make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < U; ++u) q[u] = chunk(c0 + u * NT + tid);
-    }
+    for (int u = 0; u < U; ++u) q[u] = chunk(c0 + u * NT + static_cast<int>(threadIdx.x));
   }
   // The same for one wave: chunks base + u * WAVE + lane, u < U.
   template <int U>
   __device__ __forceinline__ void wchunks(int base, float4 (&q)[U]) const {
     const int lane = threadIdx.x & (WAVE - 1);
-    if (aligned && (base + U * WAVE <= nfull || 4 * nfull == V)) {
 #pragma unroll
-      for (int u = 0; u < U; ++u) {
-        const uint4 v = buf_load16(rs, 16u * static_cast<uint32_t>(base + u * WAVE + lane), 0u);
-        q[u] = make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
-      }
-    } else {
-#pragma unroll
-      for (int u = 0; u < U; ++u) q[u] = chunk(base + u * WAVE + lane);
-    }
+    for (int u = 0; u < U; ++u) q[u] = chunk(base + u * WAVE + lane);
   }
 };
 
@@ -701,17 +672,8 @@ __device__ __forceinline__ uint32_t topk_count4(Shared32& sh, const Xform& X, in
 constexpr int TK_EARLY = FL_TK_EARLY;
 template <int U0, int U1>
 __device__ __forceinline__ void topk_tile_load(const Src& S, float4 (&q)[TK_TILE]) {
-  const int tid = threadIdx.x;
-  if (S.aligned && (U1 * NT <= S.nfull || 4 * S.nfull == S.V)) {
 #pragma unroll
-    for (int u = U0; u < U1; ++u) {
-      const uint4 v = buf_load16(S.rs, 16u * static_cast<uint32_t>(u * NT + tid), 0u);
-      q[u] = make_float4(__uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w));
-    }
-  } else {
-#pragma unroll
-    for (int u = U0; u < U1; ++u) q[u] = S.chunk(u * NT + tid);
-  }
+  for (int u = U0; u < U1; ++u) q[u] = S.chunk(u * NT + static_cast<int>(threadIdx.x));
 }
 
 // Read 1: the register tile q (keys kept in kt, the largest of chunk u in
@@ -1723,8 +1685,6 @@ __global__ __launch_bounds__(NT) void k_sample_rows32(const fl_sample_args a) {
   Src S;
   S.rs = row_rsrc(row, 4u * static_cast<uint32_t>(V));
   S.V = V;
-  S.nfull = V >> 2;
-  S.aligned = (reinterpret_cast<uintptr_t>(row) & 15u) == 0;
   // top-k rows: the first loads of the row go out before the history is read
   const bool topk_first = K > 0 && K < V && K <= TK_MAX;
   float4 q[TK_TILE];

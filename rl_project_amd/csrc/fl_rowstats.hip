@@ -9,7 +9,9 @@
 //
 // One work-group of 256 threads per row; the row streams through 16-byte
 // chunks interleaved over the threads (coalesced), 4 chunks per thread in
-// flight.  Each thread keeps, relative to its running maximum m of the row x,
+// flight.  The loads need no more than an element's alignment, so rows of an
+// odd vocabulary take them too (4096 bf16 rows of V = 50257: element by
+// element 309 us, now 132 us).  Each thread keeps, relative to its running maximum m of the row x,
 //   s = sum exp(x - m),  u = sum exp(x - m) (x - m),
 // and with a reference row y (running maximum m') also
 //   s' = sum exp(y - m'),  w = sum exp(x - m) ((x - m) - (y - m')),
@@ -145,13 +147,12 @@ __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) 
   const char* yp = KL ? static_cast<const char*>(a.ref_logits) + r * a.ref_ld * esz : xp;
   const __amdgpu_buffer_rsrc_t rx = row_rsrc(xp, static_cast<uint32_t>(V * esz));
   const __amdgpu_buffer_rsrc_t ry = row_rsrc(yp, static_cast<uint32_t>(V * esz));
-  const bool aligned = ((reinterpret_cast<uintptr_t>(xp) | reinterpret_cast<uintptr_t>(yp)) & 15u) == 0;
   const int nch = (V + N - 1) / N;
   const int nfull = V / N;
 
   Acc acc = {-__builtin_inff(), 0.0, 0.0, -__builtin_inff(), 0.0, 0.0};
   auto load = [&](__amdgpu_buffer_rsrc_t rs, int c, float (&x)[N]) __attribute__((always_inline)) {
-    if (aligned && c < nfull) {
+    if (c < nfull) {
       C::unpack(buf_load16_once(rs, 16u * c, 0u), x);  // (read once: 207 -> 201 us at 4096 x 128256 bf16)
     } else {
 #pragma unroll

@@ -164,7 +164,6 @@ struct PairRows {
   static constexpr int N = C::N;
   __amdgpu_buffer_rsrc_t rt, rd;
   fl_row_desc td, dd;
-  bool aligned;
   int V, nch, nfull;
   float cap, T;
   __device__ PairRows(const fl_spec_args& a, int64_t b, int pos) {
@@ -179,13 +178,12 @@ struct PairRows {
     const char* dp = static_cast<const char*>(a.draft) + (b * K + pos) * a.ld * esz;
     rt = row_rsrc(tp, static_cast<uint32_t>(V * esz));
     rd = row_rsrc(dp, static_cast<uint32_t>(V * esz));
-    aligned = ((reinterpret_cast<uintptr_t>(tp) | reinterpret_cast<uintptr_t>(dp)) & 15u) == 0;
     nch = (V + N - 1) / N;
     nfull = V / N;
   }
   // the raw logits of chunk c of both rows
   __device__ __forceinline__ void load(int c, float (&xt)[N], float (&xd)[N]) const {
-    if (aligned && c < nfull) {
+    if (c < nfull) {
       C::unpack(buf_load16(rt, 16u * c, 0u), xt);
       C::unpack(buf_load16(rd, 16u * c, 0u), xd);
     } else {
