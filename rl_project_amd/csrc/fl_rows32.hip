@@ -696,65 +696,37 @@ __device__ __forceinline__ void topk_read1(Shared32& sh, const Src& S, const Xfo
   });
 }
 
-// History elements (bits of the bitmap X.hbits; thread t takes words t,
-// t + NT, ...).  The first TK_HP of a thread are prefetched before read 1 and
-// kept in registers (index hi, logit hx, then z key hk); the rest, rare, are
-// loaded again by each pass that needs them.
+// History elements: thread t takes list positions t, t + NT, ...; of the
+// positions that hold one id, the first to set its bit in the bitmap claims
+// it.  A thread's first TK_HP claimed elements are fetched before read 1 and
+// kept in registers (index hi, logit hx, then z key hk); later ones (histories
+// past TK_HP * NT ids) are loaded again by each pass that needs them.  (By
+// bitmap word, a thread took all the common tokens of the lowest ids one
+// after the other: 64 rows of V = 32000 with 512 Zipf(1.1) ids 25.4 us per
+// launch, by list position 13.8 us.)
 constexpr int TK_HP = 4;
+static_assert(FL_MAX_HISTORY <= 64 * NT, "one claim bit per list position of a thread");
 struct TopkHist {
   int hi[TK_HP];
   float hx[TK_HP];
   uint32_t hk[TK_HP];
-  bool more;  // the thread's words hold more than TK_HP elements
+  uint64_t claimed;    // bit j: the thread claimed the id at position t + j NT
+  const int32_t* hid;  // the row's list
 };
 
-__device__ __forceinline__ void topk_hist_prefetch(const Src& S, const Xform& X, int V, TopkHist& h) {
-#pragma unroll
-  for (int j = 0; j < TK_HP; ++j) h.hi[j] = -1;
-  h.more = false;
-  const int nw = (V + 31) >> 5;
-  int n = 0;
-  for (int w = threadIdx.x; w < nw && !h.more; w += NT) {
-    uint32_t bits = X.hbits[w];
-    while (bits) {
-      if (n == TK_HP) {
-        h.more = true;
-        break;
-      }
-      const int i = 32 * w + __ffs(bits) - 1;
-      bits &= bits - 1u;
-#pragma unroll
-      for (int j = 0; j < TK_HP; ++j)
-        if (j == n) h.hi[j] = i;  // (static indices: the slots stay in registers)
-      ++n;
-    }
-  }
-#pragma unroll
-  for (int j = 0; j < TK_HP; ++j)
-    h.hx[j] = h.hi[j] >= 0 ? __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(S.rs, 4 * h.hi[j], 0, 0)) : 0.0f;
-}
-
-// The history elements past a thread's first TK_HP: f(i, x) for each.
+// The history elements past a thread's first TK_HP positions: f(i, x) for each.
 template <class F>
-__device__ __forceinline__ void topk_hist_rest(const Src& S, const Xform& X, int V, F&& f) {
-  const int nw = (V + 31) >> 5;
-  int n = 0;
-  for (int w = threadIdx.x; w < nw; w += NT) {
-    uint32_t bits = X.hbits[w];
-    while (bits) {
-      const int i = 32 * w + __ffs(bits) - 1;
-      bits &= bits - 1u;
-      if (n++ < TK_HP) continue;
-      f(i, __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(S.rs, 4 * i, 0, 0)));
-    }
+__device__ __forceinline__ void topk_hist_rest(const Src& S, const TopkHist& h, F&& f) {
+  for (uint64_t m = h.claimed >> TK_HP << TK_HP; m; m &= m - 1u) {
+    const int i = h.hid[threadIdx.x + NT * (__ffsll(static_cast<unsigned long long>(m)) - 1)];
+    f(i, __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(S.rs, 4 * i, 0, 0)));
   }
 }
 
 // Each history element moves from the bin of s to the bin of z = penalty(s)
 // (bad set on a NaN z); the z keys of the prefetched ones stay in h.hk.
 template <bool SC>
-__device__ __forceinline__ void topk_hist_move(Shared32& sh, const Src& S, const Xform& X, int V, TopkHist& h,
-                                               bool& bad) {
+__device__ __forceinline__ void topk_hist_move(Shared32& sh, const Src& S, const Xform& X, TopkHist& h, bool& bad) {
   auto move = [&](float x) -> uint32_t {
     const float s = topk_s<SC>(X, x);
     const float z = penalty_val<F32>(s, X.rp, X.rpr);
@@ -768,7 +740,7 @@ __device__ __forceinline__ void topk_hist_move(Shared32& sh, const Src& S, const
   };
 #pragma unroll
   for (int j = 0; j < TK_HP; ++j) h.hk[j] = h.hi[j] >= 0 ? move(h.hx[j]) : 0u;
-  if (h.more) topk_hist_rest(S, X, V, [&](int, float x) { move(x); });
+  topk_hist_rest(S, h, [&](int, float x) { move(x); });
 }
 
 // One slot per candidate: (z key << 32) | ~index, z keys turned into y keys
@@ -849,14 +821,13 @@ __device__ __forceinline__ void topk_read2(Shared32& sh, const Src& S, const Xfo
       for (int j = 0; j < TK_HP; ++j)
         if ((m >> j) & 1u) topk_put(sh, pos, h.hk[j], h.hi[j]);
     }
-    if (h.more)
-      topk_hist_rest(S, X, V, [&](int i, float x) {
-        const uint32_t kz = f32_key(penalty_val<F32>(topk_s<SC>(X, x), X.rp, X.rpr));
-        if ((kz >> TK_SH) >= kbin) {
-          uint32_t pos = atomicAdd(&sh.ncand, 1u);
-          topk_put(sh, pos, kz, i);
-        }
-      });
+    topk_hist_rest(S, h, [&](int i, float x) {
+      const uint32_t kz = f32_key(penalty_val<F32>(topk_s<SC>(X, x), X.rp, X.rpr));
+      if ((kz >> TK_SH) >= kbin) {
+        uint32_t pos = atomicAdd(&sh.ncand, 1u);
+        topk_put(sh, pos, kz, i);
+      }
+    });
   }
 }
 
@@ -876,15 +847,13 @@ __device__ __forceinline__ void topk_init(Shared32& sh) {
 // Returns false, with nothing decided, when the row needs another path.
 // Called by all threads (block-uniform control flow).
 __device__ __forceinline__ bool topk_path(Shared32& sh, const Src& S, const Xform& X, const RowCfg& R, RowOut& o,
-                                          float4 (&q)[TK_TILE]) {
+                                          float4 (&q)[TK_TILE], TopkHist& h) {
   const int tid = threadIdx.x;
   const int lane = tid & (WAVE - 1);
   const int V = R.V, K = R.K;
   if constexpr (TK_EARLY < TK_TILE) topk_tile_load<TK_EARLY, TK_TILE>(S, q);
   if (sh.status != 0) return false;  // (rows with an error status: the two-read path reports them)
   const bool sc = X.cap > 0.0f, tdiv = X.t > 0.0f;
-  TopkHist h;
-  if (X.pen) topk_hist_prefetch(S, X, V, h);
   FL_MARK(16);
   uint32_t kt[TK_TILE][4], cmx[TK_TILE];
   bool bad = false;
@@ -896,8 +865,8 @@ __device__ __forceinline__ bool topk_path(Shared32& sh, const Src& S, const Xfor
   // the adds still to come; nothing reads the bins before the barrier below)
   if (X.pen) {
     FL_MARK(10);
-    if (sc) topk_hist_move<true>(sh, S, X, V, h, bad);
-    else topk_hist_move<false>(sh, S, X, V, h, bad);
+    if (sc) topk_hist_move<true>(sh, S, X, h, bad);
+    else topk_hist_move<false>(sh, S, X, h, bad);
   }
   FL_MARK(13);
   __syncthreads();  // (every add and move before the scan reads the bins)
@@ -1702,14 +1671,40 @@ __global__ __launch_bounds__(NT) void k_sample_rows32(const fl_sample_args a) {
   if (pen) {
     for (int i = tid; i < (V + 31) / 32; i += NT) hbits_dyn[i] = 0;
   }
+  TopkHist h;
+  h.hid = hid;
+  h.claimed = 0;
+#pragma unroll
+  for (int j = 0; j < TK_HP; ++j) {
+    h.hi[j] = -1;
+    h.hx[j] = 0.0f;
+  }
   __syncthreads();
   FL_MARK(14);
   if (pen) {
-    for (int i = tid; i < H; i += NT) {
-      const int id = (hist_rows && i == tid) ? hid0 : hid[i];
-      if (id < 0 || id >= V) atomicOr(&sh.status, FL_ROW_BAD_HISTORY);
-      else atomicOr(&hbits_dyn[id >> 5], 1u << (id & 31));
+    auto claim = [&](int id) -> bool {
+      if (id < 0 || id >= V) {
+        atomicOr(&sh.status, FL_ROW_BAD_HISTORY);
+        return false;
+      }
+      const uint32_t bit = 1u << (id & 31);
+      return (atomicOr(&hbits_dyn[id >> 5], bit) & bit) == 0u;
+    };
+    int id[TK_HP];
+#pragma unroll
+    for (int j = 0; j < TK_HP; ++j) {
+      const int i = tid + j * NT;
+      id[j] = i < H ? (hist_rows && j == 0 ? hid0 : hid[i]) : 0;
     }
+#pragma unroll
+    for (int j = 0; j < TK_HP; ++j)
+      if (tid + j * NT < H && claim(id[j])) {
+        h.claimed |= 1ull << j;
+        h.hi[j] = id[j];
+        if (topk_first) h.hx[j] = __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(S.rs, 4 * id[j], 0, 0));
+      }
+    for (int j = TK_HP; tid + j * NT < H; ++j)
+      if (claim(hid[tid + j * NT])) h.claimed |= 1ull << j;
   }
   __syncthreads();
   FL_MARK(15);
@@ -1734,7 +1729,7 @@ __global__ __launch_bounds__(NT) void k_sample_rows32(const fl_sample_args a) {
   R.U = U;
   R.select = select;
   RowOut o;
-  if (!(topk_first && topk_path(sh, S, X, R, o, q)) && !two_read(sh, S, X, R, o)) {
+  if (!(topk_first && topk_path(sh, S, X, R, o, q, h)) && !two_read(sh, S, X, R, o)) {
   // ------------------------------------------------ first read: max, NaN
   uint32_t kmax = 0;
   int nan = 0;
