@@ -115,8 +115,8 @@ typedef struct fl_row_desc {
  * (slower; the same results on every other row).  Adding
  * FL_FLAG_ONLY_LIMITED repeats a call for the rows whose out_status it left
  * at FL_ROW_LIMIT and leaves every other row's outputs as they are (no host
- * synchronisation needed: the kernel reads out_status).  The Python binding
- * makes that repeat after a call that reports FL_ROW_LIMIT.
+ * synchronisation needed: the kernel reads out_status).  fl_sample_exact does
+ * both in one launch; the Python binding calls it wherever it repeats.
  */
 typedef struct fl_sample_args {
   uint32_t struct_size;        /* sizeof(fl_sample_args) */
@@ -161,6 +161,13 @@ typedef struct fl_sample_args {
  * and the return_logprobs branch of generate_tokens (sampling.py:97-98).
  */
 int fl_sample(const fl_sample_args* args, void* stream);
+
+/*
+ * fl_sample followed by the repeat for the rows it leaves at FL_ROW_LIMIT
+ * (FL_FLAG_EXACT_COUNTS | FL_FLAG_ONLY_LIMITED), in one launch: such a row's
+ * work-group samples it again.  float32 rows: fl_sample.
+ */
+int fl_sample_exact(const fl_sample_args* args, void* stream);
 
 /*
  * Materialise what apply_sampling_filters (sampling.py:16-53) returns, from

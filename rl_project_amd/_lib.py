@@ -123,6 +123,8 @@ def lib() -> ctypes.CDLL:
     handle.fl_last_error.restype = ctypes.c_char_p
     handle.fl_sample.argtypes = [ctypes.POINTER(SampleArgs), _p]
     handle.fl_sample.restype = ctypes.c_int
+    handle.fl_sample_exact.argtypes = [ctypes.POINTER(SampleArgs), _p]
+    handle.fl_sample_exact.restype = ctypes.c_int
     handle.fl_apply_filter.argtypes = [ctypes.POINTER(SampleArgs), _p, _p, ctypes.c_int64, _p, _p, _p]
     handle.fl_apply_filter.restype = ctypes.c_int
     handle.fl_spec_verify.argtypes = [ctypes.POINTER(SpecArgs), _p]
@@ -168,6 +170,6 @@ def stream_handle(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-EXPORTED_SYMBOLS = ("fl_sample", "fl_apply_filter", "fl_spec_verify", "fl_spec_verify_static",
+EXPORTED_SYMBOLS = ("fl_sample", "fl_sample_exact", "fl_apply_filter", "fl_spec_verify", "fl_spec_verify_static",
                     "fl_spec_workspace_bytes", "fl_spec_cache_workspace_bytes", "fl_lm_head_sample", "fl_lm_head_workspace_bytes", "fl_row_stats",
                     "fl_last_error", "fl_abi_version")

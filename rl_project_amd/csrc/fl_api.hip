@@ -76,20 +76,27 @@ int fl_abi_version(void) { return FL_ABI_VERSION; }
 
 const char* fl_last_error(void) { return g_error.c_str(); }
 
-int fl_sample(const fl_sample_args* a, void* stream) {
-  int rc = validate_sample(a, "fl_sample");
+namespace {
+int sample(const fl_sample_args* a, void* stream, const char* fn, bool repeat) {
+  int rc = validate_sample(a, fn);
   if (rc != FL_OK) return rc;
   const bool select = (a->flags & FL_FLAG_NO_SELECT) == 0;
-  if (select && a->out_token == nullptr) return fail(FL_EINVAL, "fl_sample: out_token is NULL");
+  if (select && a->out_token == nullptr) return fail(FL_EINVAL, "%s: out_token is NULL", fn);
   if (select && a->batch > 0 && a->uniforms == nullptr)
-    return fail(FL_EINVAL, "fl_sample: uniforms is NULL (one draw per row is required unless FL_FLAG_NO_SELECT)");
+    return fail(FL_EINVAL, "%s: uniforms is NULL (one draw per row is required unless FL_FLAG_NO_SELECT)", fn);
   if (a->batch == 0) return ok();
   // (float32 rows have no 16-bit counters: a repeat for limited rows has nothing to do)
   if (a->dtype == FL_DTYPE_F32 && (a->flags & FL_FLAG_ONLY_LIMITED)) return ok();
   const hipStream_t s = static_cast<hipStream_t>(stream);
-  const hipError_t e = a->dtype == FL_DTYPE_F32 ? fl::launch_sample_rows32(*a, s) : fl::launch_sample_rows16(*a, s);
-  return check_launch(e, "fl_sample");
+  const hipError_t e =
+      a->dtype == FL_DTYPE_F32 ? fl::launch_sample_rows32(*a, s) : fl::launch_sample_rows16(*a, s, repeat);
+  return check_launch(e, fn);
 }
+}  // namespace
+
+int fl_sample(const fl_sample_args* a, void* stream) { return sample(a, stream, "fl_sample", false); }
+
+int fl_sample_exact(const fl_sample_args* a, void* stream) { return sample(a, stream, "fl_sample_exact", true); }
 
 int fl_apply_filter(const fl_sample_args* a, const fl_row_desc* desc, void* out_filtered, int64_t out_ld,
                     float* out_probs, uint32_t* out_mask, void* stream) {

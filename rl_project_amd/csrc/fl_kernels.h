@@ -8,7 +8,9 @@
 namespace fl {
 
 // Row samplers: one work-group per row; a.dtype selects the kernel family.
-hipError_t launch_sample_rows16(const fl_sample_args& a, hipStream_t s);
+// (repeat: rows that reach FL_ROW_LIMIT are sampled again with exact counts in
+// the same launch)
+hipError_t launch_sample_rows16(const fl_sample_args& a, hipStream_t s, bool repeat);
 hipError_t launch_sample_rows32(const fl_sample_args& a, hipStream_t s);
 
 // Element-wise materialisation of filtered logits / probabilities / masks.

@@ -333,7 +333,7 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
   // (a repeat for the rows a first call left at FL_ROW_LIMIT: the others keep
   // their outputs; block-uniform, before any barrier)
   if constexpr (HEAVY)
-    if ((a.flags & FL_FLAG_ONLY_LIMITED) && (a.out_status[b] & FL_ROW_LIMIT) == 0) return true;
+    if ((a.flags & FL_FLAG_ONLY_LIMITED) && (a.out_status[b] & FL_ROW_LIMIT) == 0) return false;
   const int V = static_cast<int>(a.vocab);
   const uint16_t* row = static_cast<const uint16_t*>(a.logits) + b * a.ld;
   const bool SC_ELEM = SC && SC_ELEM_IN;
@@ -1091,15 +1091,17 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
   const bool want_cut = (a.out_desc != nullptr) && status == 0 && cut_kept < cut_total;
   float y_sel = 0.0f;
   if (want_sel || want_cut) {
-    // The row tile: the first read, still in VGPRs, or (soft-cap kernel,
-    // whose calls keep it from staying there) the row read again.  A re-read
+    // The row tile: the first read, still in VGPRs but for its last slot (whose
+    // four registers the decisions need: kept, the compiler stores a slot to
+    // scratch and loads it back), or (soft-cap kernel, whose calls keep it
+    // from staying there) the row read again.  A re-read
     // is issued here, not during the decisions: a wave stalls issuing loads
     // while the memory system is backed up, which would stall the search wave.
     uint4 r[NCH];
 #pragma unroll
     for (int j = 0; j < NCH; ++j) {
       if constexpr (SC) r[j] = fast ? buf_load16(rrow, 16u * tid, 16u * NT * j) : make_uint4(0, 0, 0, 0);
-      else if constexpr (!HEAVY) r[j] = d[j];
+      else if constexpr (!HEAVY) r[j] = j < NCH - 1 ? d[j] : buf_load16(rrow, 16u * tid, 16u * NT * j);
       else r[j] = make_uint4(0, 0, 0, 0);
     }
     // (an odd row's last value shares its dword with a value past the row,
@@ -1459,19 +1461,33 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
       a.out_desc[b] = dsc;
     }
   }
-  return true;
+  // (the same in every thread: tid 0's status above)
+  return (status & FL_ROW_LIMIT) != 0 || (want_sel && sh.result[0] < 0);
 }
 
 // The row sampler.  A row with more than 65535 equal values (a wrapped
-// 16-bit counter, seen by the entry pass) reports FL_ROW_LIMIT; the
-// exact-count kernel (FL_FLAG_EXACT_COUNTS) samples it.  (The exact body in
-// this kernel, even never run, costs every row ~6 us: the register
-// allocation of the common path gets worse.)
+// 16-bit counter, seen by the entry pass) reports FL_ROW_LIMIT; with `repeat`
+// its work-group then samples it again with the exact-count body, else the
+// exact-count kernel (FL_FLAG_EXACT_COUNTS) does when asked.  The body is a
+// function of its own, called once everything else is done: inlined, even
+// never run, it costs every row 2-6 us (the register allocation of the common
+// path gets worse), and as a kernel behind every launch it cost 256 rows
+// without any such value 1.7 us (33.9 -> 32.2 us per launch without it).
 template <class D, bool SC, bool WIDE>
-__global__ __launch_bounds__(NT) void k_sample_rows16(const fl_sample_args a, const int SC_ELEM_IN) {
+__device__ __noinline__ void exact_row(const fl_sample_args& a, const int SC_ELEM_IN, Shared16& sh) {
+  row_body<D, SC, true, WIDE>(a, SC_ELEM_IN, sh);
+}
+
+template <class D, bool SC, bool WIDE>
+__global__ __launch_bounds__(NT) void k_sample_rows16(const fl_sample_args a, const int SC_ELEM_IN, const int repeat) {
   __shared__ Shared16 sh;
   FL_MARK(11);  // (kernel entry)
-  row_body<D, SC, false, WIDE>(a, SC_ELEM_IN, sh);
+  const bool limited = row_body<D, SC, false, WIDE>(a, SC_ELEM_IN, sh);
+  if (limited && repeat) {
+    __syncthreads();  // (thread 0 has read the row's results)
+    const fl_sample_args c = a;  // (a copy: the function's reference must not keep `a` itself in memory)
+    exact_row<D, SC, WIDE>(c, SC_ELEM_IN, sh);
+  }
 }
 
 template <class D, bool SC, bool WIDE>
@@ -1481,7 +1497,7 @@ __global__ __launch_bounds__(NT) void k_sample_rows16_exact(const fl_sample_args
 }
 
 // ------------------------------------------------------------------ launch
-hipError_t launch_sample_rows16(const fl_sample_args& a, hipStream_t s) {
+hipError_t launch_sample_rows16(const fl_sample_args& a, hipStream_t s, bool repeat) {
   const bool has_pen = a.rep_penalty != nullptr && a.hist_ids != nullptr && a.hist_len != nullptr;
   const int sc_elem = (a.softcap > 0.0f && has_pen) ? 1 : 0;
   const dim3 grid(static_cast<unsigned>(a.batch)), block(NT);
@@ -1490,7 +1506,7 @@ hipError_t launch_sample_rows16(const fl_sample_args& a, hipStream_t s) {
     using D = decltype(d);
     constexpr bool SC = decltype(sc_c)::value, WIDE = decltype(wide_c)::value;
     if (a.flags & FL_FLAG_EXACT_COUNTS) hipLaunchKernelGGL((k_sample_rows16_exact<D, SC, WIDE>), grid, block, 0, s, a, sc_elem);
-    else hipLaunchKernelGGL((k_sample_rows16<D, SC, WIDE>), grid, block, 0, s, a, sc_elem);
+    else hipLaunchKernelGGL((k_sample_rows16<D, SC, WIDE>), grid, block, 0, s, a, sc_elem, repeat ? 1 : 0);
   };
   auto launch_w = [&](auto d, auto sc_c) {
     if (wide) launch(d, sc_c, std::true_type{});

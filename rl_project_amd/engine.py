@@ -140,11 +140,7 @@ class BatchedSampler:
         call.args.logits = logits.data_ptr()
         call.args.uniforms = uniforms.data_ptr()
         call.keep = (logits, uniforms)   # alive until the kernel has read them
-        call.run()
-        # 16-bit rows where one value fills more than 65535 positions: the
-        # exact-count repeat (a kernel that leaves every other row alone)
-        if logits.size(1) > 0xFFFF:
-            call.run_exact_for_limited()
+        call.run_exact()
         return SampleOutput(call.tokens, call.finished[:n].view(torch.bool), call.status, call.logprob)
 
     def _step_slots(self, logits, uniforms, return_logprobs, slots) -> SampleOutput:
@@ -158,9 +154,7 @@ class BatchedSampler:
         call = _Call(logits, temperature=self.temperature[idx], top_k=self.top_k[idx], top_p=self.top_p[idx],
                      min_p=self.min_p[idx], repetition_penalty=self.rep_penalty[idx], history=(hist, hlen),
                      stop_ids=self.stop_ids[idx], uniforms=uniforms, finished=fin, out_finished=fin,
-                     flags=_lib.FL_FLAG_APPEND_HISTORY, want_logprob=return_logprobs).run()
-        if logits.size(1) > 0xFFFF:
-            call.run_exact_for_limited()
+                     flags=_lib.FL_FLAG_APPEND_HISTORY, want_logprob=return_logprobs).run_exact()
         self.history.index_copy_(0, idx, hist)
         self.hist_len.index_copy_(0, idx, hlen)
         self.finished_u8.index_copy_(0, idx, fin)
