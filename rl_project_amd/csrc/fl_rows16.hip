@@ -48,6 +48,7 @@ constexpr int EARLY_CHUNKS = 4;                  // row chunks per thread reques
 #endif
 constexpr int LOOKAHEAD = FL_LOOKAHEAD;          // row chunks per thread in flight while counting
 static_assert(LOOKAHEAD >= EARLY_CHUNKS && LOOKAHEAD <= NCH, "lookahead window");
+constexpr int SHORT_MAX = 512;                   // entries one wave decides over
 constexpr int XSLOTS = 4;                        // slots past the tile in flight
 constexpr int MAX_HEAVY = 8;                     // patterns with more than 65535 values (at most 5 exist)
 
@@ -74,6 +75,8 @@ struct Shared16 {
   } dec;  // results of the search wave
   uint32_t wc[2][NSLOT][NWAVE];  // identification: members per slot of NT chunks and wave
   uint32_t nh[2];         // identification: history members
+  uint32_t short_tot;     // values in the entries of a row decided by one wave
+  int32_t short_ok;       // the wave has decided the row
   uint32_t inf_extra;     // soft-capped rows: -inf values beyond their pattern's 16-bit count
   // patterns with more than 65535 values (at most 5: V + unique history ids
   // <= 327680): their order, exact count and the part beyond the 16-bit field
@@ -399,6 +402,8 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
     sh.status = 0;
     sh.nh[0] = sh.nh[1] = 0;
     sh.n_heavy = 0;
+    sh.short_tot = 0;
+    sh.short_ok = 0;
     sh.result[0] = sh.result[1] = -1;
     sh.dec.L = 0;
     sh.dec.i0 = -1;
@@ -820,7 +825,220 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
   }
   auto Y = [&](int i) -> float { return cached ? Yc[i] : y_raw(i); };
   auto E = [&](int i) -> float { return cached ? Ec[i] : exp_of_order<D, SC>(ent[i] >> 16, CAP, T, RT, sc_entry, M); };
-  {
+  const int lane = tid & (WAVE - 1);
+  // ---------------- short lists: one wave decides
+  // Every decision of a top-k row (a request's default keeps 50) acts on the
+  // entries down to its K-th value, at most K and the run equal to it, and a
+  // short row has few entries to begin with.  For up to SHORT_MAX of them, wave
+  // 0 takes all the decisions with wave scans, in the arithmetic of the block
+  // phases below (integer sums: the same results bit for bit), while the other
+  // waves sum the counts of all entries for the total's check.  The phases of
+  // a long list are chains of block barriers and two dozen LDS round trips:
+  // 1 bf16 row of V = 128256 under top-k 50, 26.6 -> 22.9 us per launch; 37
+  // f16 rows of V = 151936 (~20 thousand distinct values), 42.7 -> 26.9 us.
+  bool done = false;
+  if constexpr (!HEAVY) {
+    const bool tk = K > 0 && K < V;
+    if (N > 0 && (N <= SHORT_MAX || (tk && K <= SHORT_MAX))) {  // block-uniform
+      if (tid < WAVE) {
+        float* const Ys = reinterpret_cast<float*>(sh.hist + SLICE_BASE);
+        float* const Es = Ys + SHORT_MAX;
+        uint32_t* const Cs = sh.hist + SLICE_BASE + 2 * SHORT_MAX;                              // n + 1 counts
+        uint64_t* const Ms = reinterpret_cast<uint64_t*>(sh.hist + SLICE_BASE + 3 * SHORT_MAX + 2);  // n + 1 masses
+        static_assert(SLICE_BASE % 2 == 0 && 5 * SHORT_MAX + 4 <= 3 * NT, "the lists fit past the entries");
+        int n = N;
+        if (tk) {
+          int ik = N;
+          uint32_t run = 0;
+          for (int i0 = 0; i0 < N && ik == N; i0 += WAVE) {  // (every entry counts at least one value)
+            const int i = i0 + lane;
+            const uint32_t inc = wave_incl_scan(i < N ? cnt_of(i) : 0u);
+            const uint64_t m = __ballot(i < N && run + inc >= static_cast<uint32_t>(K));
+            if (m) ik = i0 + __ffsll(static_cast<unsigned long long>(m)) - 1;
+            run += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(inc), WAVE - 1));
+          }
+          if (ik < N) {  // the entries down to the last that equals the K-th value
+            const float yk = y_raw(ik);
+            for (int i0 = ik + 1; i0 < N && n == N && i0 <= SHORT_MAX; i0 += WAVE) {
+              const int i = i0 + lane;
+              const uint64_t m = __ballot(i < N && y_raw(i) < yk);
+              if (m) n = i0 + __ffsll(static_cast<unsigned long long>(m)) - 1;
+            }
+          }
+        }
+        if (n <= SHORT_MAX) {
+          // values, weights and exclusive prefixes
+          uint32_t rc = 0;
+          uint64_t rm = 0;
+          for (int i0 = 0; i0 < n; i0 += WAVE) {
+            const int i = i0 + lane;
+            uint32_t c = 0;
+            uint64_t m = 0;
+            if (i < n) {
+              const float y = y_raw(i), e = expf(y - M);
+              Ys[i] = y;
+              Es[i] = e;
+              c = cnt_of(i);
+              m = c * to_fx(e);
+            }
+            const uint32_t ic = wave_incl_scan(c);
+            const uint64_t im = wave_incl_scan(m);
+            if (i < n) {
+              Cs[i + 1] = rc + ic;
+              Ms[i + 1] = rm + im;
+            }
+            rc += static_cast<uint32_t>(__builtin_amdgcn_readlane(static_cast<int>(ic), WAVE - 1));
+            rm += readlane64(im, WAVE - 1);
+          }
+          if (lane == 0) {
+            Cs[0] = 0;
+            Ms[0] = 0;
+          }
+          __builtin_amdgcn_wave_barrier();
+          // first i in [0, m) with pred(i, ex), ex = the sum of term before i
+          // (m when none; *ex_out: the sum before the result)
+          auto scan = [&](int m, auto&& term, auto&& pred, uint64_t* ex_out) -> int {
+            uint64_t carry = 0;
+            for (int i0 = 0; i0 < m; i0 += WAVE) {
+              const int i = i0 + lane;
+              const uint64_t v = i < m ? term(i) : 0ull;
+              const uint64_t inc = wave_incl_scan(v);
+              const uint64_t ex = carry + inc - v;
+              const uint64_t hit = __ballot(i < m && pred(i, ex));
+              if (hit) {
+                const int f = __ffsll(static_cast<unsigned long long>(hit)) - 1;
+                *ex_out = readlane64(ex, f);
+                return i0 + f;
+              }
+              carry += readlane64(inc, WAVE - 1);
+            }
+            *ex_out = carry;
+            return m;
+          };
+          auto glo = [&](int i, float y) { return wave_first(0, i + 1, [&](int j) { return Ys[j] <= y; }); };
+          auto ghi = [&](int i, float y) { return wave_first(i + 1, n, [&](int j) { return Ys[j] < y; }) - 1; };
+          // min-p (the list ends where top-k does)
+          int L = n;
+          double S = from_fx(Ms[L]);
+          if (MP > 0.0f) {
+            const float r = 1.0f / static_cast<float>(S);
+            const float thr = D::rn(D::rn(r) * MP);
+            L = wave_first(0, n, [&](int i) { return D::rn(Es[i] * r) < thr; });
+            S = from_fx(Ms[L]);
+          }
+          // top-p
+          int ic = L - 1;
+          uint32_t nc = L > 0 ? cnt_of(L - 1) : 0u;
+          const float r1 = 1.0f / static_cast<float>(S);
+          if (L > 0 && TP > 0.0f && TP < 1.0f) {
+            const float t = D::rn(TP);
+            auto removed = [&](uint64_t c_incl, float p) {
+              return D::rn(D::rn(static_cast<float>(from_fx(c_incl))) - p) >= t;
+            };
+            uint64_t ex;
+            const int x = scan(L, [&](int i) { return cnt_of(i) * to_fx(D::rn(Es[i] * r1)); },
+                               [&](int i, uint64_t e) {
+                                 const float p = D::rn(Es[i] * r1);
+                                 return removed(e + to_fx(p), p);
+                               }, &ex);
+            ic = x - 1;
+            if (ic >= 0) {
+              const float p = D::rn(Es[ic] * r1);
+              const uint64_t pfi = to_fx(p), c = ex - cnt_of(ic) * pfi;
+              nc = static_cast<uint32_t>(wave_first(1, static_cast<int>(cnt_of(ic)), [&](int j) {
+                return removed(c + static_cast<uint64_t>(j + 1) * pfi, p);
+              }));
+            }
+          }
+          if (L > 0 && ic >= 0) {
+            const float ycut = Ys[ic];
+            const int cut_lo = glo(ic, ycut), cut_hi = ghi(ic, ycut);
+            const uint32_t nk = Cs[ic] + nc;
+            const double SKs = from_fx(Ms[ic] + nc * to_fx(Es[ic]));
+            if (lane == 0) {
+              sh.dec.cut_total = Cs[cut_hi + 1] - Cs[cut_lo];
+              sh.dec.cut_kept = nk - Cs[cut_lo];
+              sh.dec.cut_lo = cut_lo;
+              sh.dec.cut_hi = cut_hi;
+              sh.dec.n_kept = nk;
+              sh.dec.SK = SKs;
+              sh.dec.y_cut = ycut;
+              sh.dec.o_lo[1] = ent[cut_lo] >> 16;
+              sh.dec.o_hi[1] = ent[cut_hi] >> 16;
+            }
+            const float rKs = 1.0f / static_cast<float>(SKs);
+            auto q_of = [&](int i) { return D::rn(Es[i] * rKs); };
+            auto kcs = [&](int i) -> uint32_t { return i < ic ? cnt_of(i) : nc; };
+            int g = 0, g_hi = 0;
+            uint32_t rank = 0;
+            if (select && T <= 0.0f) {  // greedy: first index among the maximal probabilities
+              const float qmax = q_of(0);
+              const int last = wave_first(1, ic + 1, [&](int i) { return q_of(i) != qmax; }) - 1;
+              g_hi = ghi(last, Ys[last]);
+            } else if (select) {        // inverse CDF
+              // (the kept q-mass prefixes take the place of the masses)
+              uint64_t run = 0;
+              for (int i0 = 0; i0 <= ic; i0 += WAVE) {
+                const int i = i0 + lane;
+                const uint64_t inc = run + wave_incl_scan(i <= ic ? kcs(i) * to_fx(q_of(i)) : 0ull);
+                if (i <= ic) Ms[i + 1] = inc;
+                run = readlane64(inc, WAVE - 1);
+              }
+              __builtin_amdgcn_wave_barrier();
+              // (an opaque copy: otherwise the conversion of U is shared with the
+              // block phases, held in two VGPRs from the kernel's start, and a
+              // chunk of the row tile goes to scratch for it)
+              float us = U;
+              asm volatile("" : "+v"(us));
+              const uint64_t target = __double2ull_rd(static_cast<double>(us) * static_cast<double>(run));
+              int is = wave_first(0, ic + 1, [&](int i) { return Ms[i + 1] > target; });
+              if (is > ic) is = 0;  // every kept probability rounds to zero
+              const float ys = Ys[is];
+              g = glo(is, ys);
+              g_hi = ghi(is, ys);
+              const uint64_t cg = Ms[g];
+              const uint64_t q = to_fx(q_of(is));
+              const uint32_t kept_g = (g_hi + 1 <= ic ? Cs[g_hi + 1] : nk) - (g <= ic ? Cs[g] : nk);
+              // member r covers [cg + r q, cg + (r + 1) q): the first whose end
+              // passes the target (the last kept one if none does)
+              if (q > 0 && target >= cg && kept_g > 0)
+                rank = static_cast<uint32_t>(wave_first(0, static_cast<int>(kept_g) - 1, [&](int r) {
+                  return cg + static_cast<uint64_t>(r + 1) * q > target;
+                }));
+            }
+            if (lane == 0) {
+              sh.dec.sel_rank = rank;
+              sh.dec.y_sel = Ys[g];
+              sh.dec.o_lo[0] = ent[g] >> 16;
+              sh.dec.o_hi[0] = ent[g_hi] >> 16;
+            }
+          }
+          if (lane == 0) {
+            sh.dec.L = L;
+            sh.dec.S = S;
+            sh.dec.i0 = ic;
+            sh.dec.c0 = nc;
+            sh.short_ok = 1;
+          }
+        }
+      } else {
+        uint32_t c = 0;
+        for (int i = tid - WAVE; i < N; i += NT - WAVE) c += cnt_of(i);
+        c = wave_reduce(c, OpAdd());
+        if (lane == 0 && c) atomicAdd(&sh.short_tot, c);
+      }
+      __syncthreads();
+      done = sh.short_ok != 0;
+      if (done) {
+        // (a total other than V less the -inf values: a wrapped 16-bit counter)
+        const uint32_t tc = sh.short_tot;
+        if (tc != static_cast<uint32_t>(V) && tc + neg_inf_count() != static_cast<uint32_t>(V) && tid == 0)
+          atomicOr(&sh.status, FL_ROW_LIMIT);
+        lds_barrier();  // (every wave past the counts and flags before the status is read)
+      }
+    }
+  }
+  if (!done) {
     uint32_t lc = 0;
     uint64_t lm = 0;
     for (int i = lo; i < hi; ++i) {
@@ -860,7 +1078,7 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
     if (tid == 0 && tc != static_cast<uint32_t>(V) && tc + neg_inf_count() != static_cast<uint32_t>(V))
       atomicOr(&sh.status, FL_ROW_LIMIT);
   }
-  __syncthreads();
+  if (!done) __syncthreads();
   int32_t status = sh.status;
   FL_MARK(4);
 
@@ -878,7 +1096,6 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
     for (int i = s * per; i < L; ++i) m += cnt_of(i) * to_fx(E(i));
     return m;
   };
-  const int lane = tid & (WAVE - 1);
   // Entries of equal value Y form a group (several patterns can round to one
   // value).  Y is non-increasing along the entries, so a group is a run; the
   // window of 64 entries next to i settles its bound in one probe unless the
@@ -904,7 +1121,7 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
   const bool w0 = tid < WAVE;
 
   // ---------------- top-k (sampling.py:36-38) and min-p (:40-43): value cuts
-  if (status == 0) {
+  if (status == 0 && !done) {
     if (w0) {
       int L = N;
       if (K > 0 && K < V) {
@@ -944,7 +1161,7 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
   // predicate is monotone along the order, so the kept set is a prefix: a
   // block scan finds the first removed entry (tested on its first member),
   // then wave 0 counts the kept members of the entry before it.
-  if (status == 0) {
+  if (status == 0 && !done) {
     const double S = sh.dec.S;
     int i0 = L - 1;
     uint32_t c0 = cnt_of(L - 1);
@@ -1008,7 +1225,7 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
   const int i0 = sh.dec.i0;
   const uint32_t c0 = sh.dec.c0;
   if (status == 0 && i0 < 0) status |= FL_ROW_ALL_MASKED;
-  const double SK = sh.dec.SK;
+  const double SK = status == 0 ? sh.dec.SK : 0.0;  // (one wave may have decided a row that has a status)
   const float rK = 1.0f / static_cast<float>(SK);
   const uint32_t n_kept = sh.dec.n_kept;
   const uint32_t cut_kept = sh.dec.cut_kept, cut_total = sh.dec.cut_total;
@@ -1018,7 +1235,7 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
   auto kc = [&](int i) -> uint32_t { return i < i0 ? cnt_of(i) : (i == i0 ? c0 : 0u); };
   auto kept_before = [&](int Lb) -> uint32_t { return Lb <= i0 ? count_before(Lb) : n_kept; };
   const bool want_sel = select && status == 0;
-  if (want_sel) {
+  if (want_sel && !done) {
     if (T <= 0.0f) {
       // greedy (sampling.py:59-60): first index among the maximal probabilities
       if (w0) {
@@ -1104,21 +1321,12 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
       else if constexpr (!HEAVY) r[j] = j < NCH - 1 ? d[j] : buf_load16(rrow, 16u * tid, 16u * NT * j);
       else r[j] = make_uint4(0, 0, 0, 0);
     }
-    // (an odd row's last value shares its dword with a value past the row,
-    // which the range check turns to zeros whole: it is read by itself)
-    if (!WIDE && (V & 1) && fast) {
-      const int jl = nfull / NT;
-      const uint32_t last = tid == nfull % NT ? static_cast<uint32_t>(row[V - 1]) : 0u;
-      const int wl = ((V - 1) & 7) >> 1;
+    // the owned prefetched ids, read again in time for their member tests
+    // (held in VGPRs through the decisions, they would push a chunk of the row
+    // tile out to scratch)
+    int32_t hown[HPRE];
 #pragma unroll
-      for (int j = 0; j < NCH; ++j)
-        if (j == jl) {  // (block-uniform, as is wl)
-          r[j].x |= wl == 0 ? last : 0u;
-          r[j].y |= wl == 1 ? last : 0u;
-          r[j].z |= wl == 2 ? last : 0u;
-          r[j].w |= wl == 3 ? last : 0u;
-        }
-    }
+    for (int k = 0; k < HPRE; ++k) hown[k] = own[k] ? hid[tid + k * NT] : 0;
     lds_barrier();  // the decisions are in sh.dec; the entries may be overwritten
     FL_MARK(13);
     y_sel = sh.dec.y_sel;
@@ -1200,8 +1408,10 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
     const int wv = __builtin_amdgcn_readfirstlane(tid / WAVE);
     const int lane_id = tid & (WAVE - 1);
     // the partial chunk (V not a multiple of 8): its zero padding reads as
-    // the pattern of +0.0
-    const int pad = (nfull < nchunks) ? 8 - (V - nfull * 8) : 0;
+    // the pattern of +0.0, and so does the last value of an odd row, whose
+    // dword reaches past the row (the range check works dword by dword): that
+    // value is tested by itself
+    const int pad = (nfull < nchunks) ? 8 - (V - nfull * 8) + (V & 1) : 0;
     const uint32_t ones2 = 0x00010001u;
 #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -1259,11 +1469,10 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
             q[k] = buf_load16(rrow, 16u * static_cast<uint32_t>(tid + (j0 + k) * NT), 0u);
 #pragma unroll
           for (int k = 0; k < XSLOTS; ++k) {
-            const int c = (j0 + k) * NT + tid;
-            if (c == nfull) q[k] = load_chunk16(row, c, V);  // (an odd row's last value, as above)
             if (j0 + k < nslots) member_test(q[k], j0 + k);
           }
         }
+        if ((V & 1) && tid == nfull % NT && in_range(t, row[V - 1])) atomicAdd(&sh.wc[t][nfull / NT][wv], 1u);
         // +0.0 a target: take back the zeros of the padding and of the lanes
         // past the row
         if (zero_in && lane_id == 0) {
@@ -1301,7 +1510,7 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
       for (int k = 0; k < HPRE; ++k)
         if (own[k]) {
           const uint32_t z = (hz >> (16 * k)) & 0xFFFFu;
-          hist_candidate(hpre[k], z, penalised_bits<D>(z, RP));
+          hist_candidate(hown[k], z, penalised_bits<D>(z, RP));
         }
       // (wide rows claimed every id in the windowed pass: none was prefetched)
       for (int i = tid + ((hist_rows && !wide && !HEAVY) ? HPRE * NT : 0); i < H; i += NT) {
@@ -1359,6 +1568,7 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
 #pragma unroll
                 for (int j = 0; j < NCH; ++j)
                   if (j == js) q = r[j];  // js is wave-uniform
+                if (c == nfull) q = load_chunk16(row, c, V);  // (the partial chunk, an odd row's last value)
               } else {
                 q = load_chunk16(row, c, V);
               }
