@@ -170,6 +170,23 @@ int fl_sample(const fl_sample_args* args, void* stream);
 int fl_sample_exact(const fl_sample_args* args, void* stream);
 
 /*
+ * The parameter arrays of a call whose rows all use the same values: out
+ * (6 * batch 4-byte words, 4-byte aligned device memory) holds temperature,
+ * top_k, top_p, min_p, rep_penalty and hist_len, `batch` entries each, in that
+ * order.
+ */
+typedef struct fl_row_values {
+  float temperature;
+  int32_t top_k;
+  float top_p;
+  float min_p;
+  float rep_penalty;
+  int32_t hist_len;
+} fl_row_values;
+
+int fl_fill_rows(const fl_row_values* values, int64_t batch, void* out, void* stream);
+
+/*
  * Materialise what apply_sampling_filters (sampling.py:16-53) returns, from
  * the descriptors of a previous fl_sample call on the same args:
  *   out_filtered[b, i] = kept ? y_i : -inf   (logits dtype, row stride out_ld)

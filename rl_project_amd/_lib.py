@@ -56,6 +56,13 @@ class SampleArgs(ctypes.Structure):
     ]
 
 
+class RowValues(ctypes.Structure):
+    _fields_ = [
+        ("temperature", ctypes.c_float), ("top_k", ctypes.c_int32), ("top_p", ctypes.c_float),
+        ("min_p", ctypes.c_float), ("rep_penalty", ctypes.c_float), ("hist_len", ctypes.c_int32),
+    ]
+
+
 class SpecArgs(ctypes.Structure):
     _fields_ = [
         ("struct_size", ctypes.c_uint32), ("dtype", ctypes.c_int32),
@@ -125,6 +132,8 @@ def lib() -> ctypes.CDLL:
     handle.fl_sample.restype = ctypes.c_int
     handle.fl_sample_exact.argtypes = [ctypes.POINTER(SampleArgs), _p]
     handle.fl_sample_exact.restype = ctypes.c_int
+    handle.fl_fill_rows.argtypes = [ctypes.POINTER(RowValues), ctypes.c_int64, _p, _p]
+    handle.fl_fill_rows.restype = ctypes.c_int
     handle.fl_apply_filter.argtypes = [ctypes.POINTER(SampleArgs), _p, _p, ctypes.c_int64, _p, _p, _p]
     handle.fl_apply_filter.restype = ctypes.c_int
     handle.fl_spec_verify.argtypes = [ctypes.POINTER(SpecArgs), _p]
@@ -170,6 +179,6 @@ def stream_handle(device: torch.device) -> int:
     return torch.cuda.current_stream(device).cuda_stream
 
 
-EXPORTED_SYMBOLS = ("fl_sample", "fl_sample_exact", "fl_apply_filter", "fl_spec_verify", "fl_spec_verify_static",
+EXPORTED_SYMBOLS = ("fl_sample", "fl_sample_exact", "fl_fill_rows", "fl_apply_filter", "fl_spec_verify", "fl_spec_verify_static",
                     "fl_spec_workspace_bytes", "fl_spec_cache_workspace_bytes", "fl_lm_head_sample", "fl_lm_head_workspace_bytes", "fl_row_stats",
                     "fl_last_error", "fl_abi_version")

@@ -98,6 +98,15 @@ int fl_sample(const fl_sample_args* a, void* stream) { return sample(a, stream, 
 
 int fl_sample_exact(const fl_sample_args* a, void* stream) { return sample(a, stream, "fl_sample_exact", true); }
 
+int fl_fill_rows(const fl_row_values* v, int64_t batch, void* out, void* stream) {
+  if (v == nullptr) return fail(FL_EINVAL, "fl_fill_rows: values is NULL");
+  if (batch < 0 || batch > 0x7fffffff)
+    return fail(FL_EINVAL, "fl_fill_rows: bad batch %lld", static_cast<long long>(batch));
+  if (batch == 0) return ok();
+  if (out == nullptr) return fail(FL_EINVAL, "fl_fill_rows: out is NULL");
+  return check_launch(fl::launch_fill_rows(*v, batch, out, static_cast<hipStream_t>(stream)), "fl_fill_rows");
+}
+
 int fl_apply_filter(const fl_sample_args* a, const fl_row_desc* desc, void* out_filtered, int64_t out_ld,
                     float* out_probs, uint32_t* out_mask, void* stream) {
   int rc = validate_sample(a, "fl_apply_filter");

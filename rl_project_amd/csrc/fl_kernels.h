@@ -13,6 +13,9 @@ namespace fl {
 hipError_t launch_sample_rows16(const fl_sample_args& a, hipStream_t s, bool repeat);
 hipError_t launch_sample_rows32(const fl_sample_args& a, hipStream_t s);
 
+// One value per parameter, written to every row's entry.
+hipError_t launch_fill_rows(const fl_row_values& v, int64_t batch, void* out, hipStream_t s);
+
 // Element-wise materialisation of filtered logits / probabilities / masks.
 hipError_t launch_apply_filter(const fl_sample_args& a, const fl_row_desc* desc, void* out_filtered, int64_t out_ld,
                                float* out_probs, uint32_t* out_mask, hipStream_t s);

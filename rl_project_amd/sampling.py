@@ -73,8 +73,48 @@ def _per_row(value: PerRow, B: int, dtype: torch.dtype, device: torch.device, of
     return t.contiguous()
 
 
-def _history_tensor(history, B: int, V: int, device: torch.device) -> Tuple[Optional[torch.Tensor], Optional[torch.Tensor], int]:
-    """Pack per-row histories into ([B, H] int32, [B] int32 lengths, row stride)."""
+_F32_MAX = 3.4028234663852886e38
+
+
+def _same_for_all(value, off) -> Optional[Union[int, float]]:
+    """The one value of a parameter given as a scalar (``off`` for None) that a
+    float32 or int32 holds without overflow, else None."""
+    if value is None:
+        return off
+    if type(value) is float:
+        return value if type(off) is float and abs(value) <= _F32_MAX else None
+    if type(value) is int:
+        return value if -(1 << 31) <= value < (1 << 31) else None
+    return None
+
+
+def _param_arrays(params, hist_len: Optional[int], B: int, device: torch.device) -> List[torch.Tensor]:
+    """The per-row arrays of temperature, top_k, top_p, min_p and
+    repetition_penalty, given as (value, dtype, off) each, and the history
+    lengths when every row's is ``hist_len``.  Parameters given as scalars are
+    written by one launch (a fill each took 5 to 6 launches a call)."""
+    same = [_same_for_all(v, off) for v, _, off in params]
+    block = None
+    if B > 0 and sum(v is not None for v in same) + (hist_len is not None) > 1:
+        block = torch.empty(6, B, dtype=torch.int32, device=device)
+        vals = [off if v is None else v for v, (_, _, off) in zip(same, params)]
+        check(lib().fl_fill_rows(_lib.RowValues(*vals, hist_len or 0), B, block.data_ptr(),
+                                 _lib.stream_handle(device)), "fl_fill_rows")
+    out = []
+    for j, (v, dt, off) in enumerate(params):
+        if block is not None and same[j] is not None:
+            out.append(block[j] if dt == torch.int32 else block[j].view(dt))
+        else:
+            out.append(_per_row(v, B, dt, device, off))
+    if hist_len is not None:
+        out.append(block[5] if block is not None else torch.full((B,), hist_len, dtype=torch.int32, device=device))
+    return out
+
+
+def _history_tensor(history, B: int, V: int, device: torch.device,
+                    lengths: bool = True) -> Tuple[Optional[torch.Tensor], Optional[torch.Tensor], int]:
+    """Pack per-row histories into ([B, H] int32, [B] int32 lengths, row
+    stride); without ``lengths`` they are None where every row's is H."""
     if history is None:
         return None, None, 0
     if (isinstance(history, tuple) and len(history) == 2 and isinstance(history[0], torch.Tensor)
@@ -93,7 +133,7 @@ def _history_tensor(history, B: int, V: int, device: torch.device) -> Tuple[Opti
         if h.dim() == 1:
             h = h.unsqueeze(0).expand(B, -1)
         h = h.contiguous()
-        lens = torch.full((B,), h.size(1), dtype=torch.int32, device=device)
+        lens = torch.full((B,), h.size(1), dtype=torch.int32, device=device) if lengths else None
         return h, lens, h.size(1)
     rows: List[List[int]] = [list(r) if r is not None else [] for r in history]
     if len(rows) != B:
@@ -143,12 +183,13 @@ class _Call:
         B, V = logits.shape
         dev = logits.device
         self.B, self.V = B, V
-        self.T = _per_row(temperature, B, torch.float32, dev, 1.0)
-        self.K = _per_row(top_k, B, torch.int32, dev, 0)
-        self.P = _per_row(top_p, B, torch.float32, dev, 1.0)
-        self.MP = _per_row(min_p, B, torch.float32, dev, 0.0)
-        self.RP = _per_row(repetition_penalty, B, torch.float32, dev, 1.0)
-        self.hist, self.hist_len, self.hist_ld = _history_tensor(history, B, V, dev)
+        self.hist, self.hist_len, self.hist_ld = _history_tensor(history, B, V, dev, lengths=False)
+        same_len = self.hist.size(1) if self.hist is not None and self.hist_len is None else None
+        self.T, self.K, self.P, self.MP, self.RP, *lens = _param_arrays(
+            ((temperature, torch.float32, 1.0), (top_k, torch.int32, 0), (top_p, torch.float32, 1.0),
+             (min_p, torch.float32, 0.0), (repetition_penalty, torch.float32, 1.0)), same_len, B, dev)
+        if lens:
+            self.hist_len = lens[0]
         self.stop, self.stop_ld, self.n_stop = _stop_tensor(stop_ids, B, dev)
         select = not (flags & FL_FLAG_NO_SELECT)
         uniform_div = max(1, int(uniform_div))
@@ -238,7 +279,7 @@ class SamplerPlan:
 
 
 def _raise_on_status(status: torch.Tensor, allowed: int = 0) -> None:
-    bad = status & ~allowed
+    bad = status.cpu() & ~allowed   # (one copy to the host; the tests on the GPU were three launches)
     if bool((bad != 0).any()):
         rows = torch.nonzero(bad).flatten().tolist()
         codes = 0
@@ -279,6 +320,8 @@ def sample_tokens(
     Equivalent to ``engine.py:118-127`` applied to every row: the filtered
     logits of ``apply_sampling_filters``, ``sample_from_logits``, the stop test
     and (``return_logprobs``) the post-filter log-probability of the token."""
+    if finished is not None and finished.dtype == torch.bool and finished.is_contiguous():
+        finished = finished.view(torch.uint8)   # (a flag is a byte of 0 or 1 in both types: no conversion)
     call = _Call(logits, temperature=temperature, top_k=top_k, top_p=top_p, min_p=min_p,
                  repetition_penalty=repetition_penalty, history=history, stop_ids=stop_ids, uniforms=uniforms,
                  finished=finished, softcap=softcap, flags=0, want_logprob=return_logprobs,
@@ -288,7 +331,7 @@ def sample_tokens(
         _raise_on_status(call.status)
     else:
         call.run()
-    return SampleOutput(call.tokens, call.finished.bool(), call.status, call.logprob, call.desc)
+    return SampleOutput(call.tokens, call.finished.view(torch.bool), call.status, call.logprob, call.desc)
 
 
 def describe_rows(logits: torch.Tensor, **kw) -> Tuple[torch.Tensor, torch.Tensor]:
@@ -322,6 +365,15 @@ def _normalise_past(past_tokens: Optional[Sequence[int]], V: int) -> Optional[Li
     wrap once, anything else outside [0, V) is an IndexError."""
     if not past_tokens:
         return None
+    if isinstance(past_tokens, list) and type(past_tokens[0]) is int:
+        try:
+            t = torch.tensor(past_tokens, dtype=torch.int64)
+        except (TypeError, ValueError, RuntimeError, OverflowError):
+            t = None   # (something that is not a number: the loop below says so)
+        if t is not None and t.dim() == 1:
+            lo, hi = (int(v) for v in torch.aminmax(t))
+            if lo >= 0 and hi < V:
+                return past_tokens
     ids = []
     for t in past_tokens:
         t = int(t)
