@@ -7,21 +7,24 @@
 //                           (src/forgeline/training/common/logprobs.py:58-62)
 // all in float32 as the reference's .float() computes them.
 //
-// One work-group of 256 threads per row; the row streams through 16-byte
-// chunks interleaved over the threads (coalesced), 4 chunks per thread in
-// flight.  The loads need no more than an element's alignment, so rows of an
-// odd vocabulary take them too (4096 bf16 rows of V = 50257: element by
-// element 309 us, now 132 us).  Each thread keeps, relative to its running maximum m of the row x,
+// One work-group per row; the row streams through 16-byte chunks interleaved
+// over the threads (coalesced), 2 chunks per thread in flight.  The loads need
+// no more than an element's alignment, so rows of an odd vocabulary take them
+// too (4096 bf16 rows of V = 50257: element by element 309 us, so 132 us).  Each thread keeps, relative to a reference m
+// near its maximum of the row x,
 //   s = sum exp(x - m),  u = sum exp(x - m) (x - m),
-// and with a reference row y (running maximum m') also
+// and with a reference row y (its m') also
 //   s' = sum exp(y - m'),  w = sum exp(x - m) ((x - m) - (y - m')),
-// in float64, rescaled when a maximum grows.  The partials merge in a fixed
-// tree, so results are deterministic.  With M, S the row's maximum and sum:
+// in float64, rescaled when m moves.  The partials are added in a fixed tree
+// once all are relative to the row's largest m, so results are deterministic.
+// With M that reference and S the row's sum:
 //   log p(label) = x_label - M - log S
 //   entropy      = log S - u / S
 //   KL           = w / S - log S + log S'
 // A -inf logit contributes exp(-inf) * (-inf) = NaN to u and w, as 0 * -inf
 // does in the reference's expression.
+#include <type_traits>
+
 #include "fl_device.h"
 #include "fl_kernels.h"
 
@@ -29,10 +32,15 @@ namespace fl {
 
 namespace {
 
-constexpr int NT_RS = 256;
-constexpr int NW_RS = NT_RS / WAVE;
 constexpr float LOG2E_F = 1.44269504088896340736f;
 constexpr double LN2_D = 0.69314718055994530942;
+// A thread moves its reference m only once a value passes it by more than
+// this: a re-base is a double-precision exponential, and while every new
+// maximum took one, some lane of a wave had one in nearly every iteration
+// (4096 bf16 rows of V = 128256: 195 us, without it 188 us).  Terms stay below
+// e^8, far from any float's range, and every sum is relative to m whatever
+// m is.
+constexpr float SLACK = 8.0f;
 
 template <class D>
 struct RowChunk;
@@ -71,10 +79,10 @@ struct RowChunk<F16> : RowChunk16<F16> {};
 
 // Running state of one row for one thread (or a merged set of threads).
 struct Acc {
-  float m;    // running maximum of x (-inf: nothing yet)
+  float m;    // reference of x, its maximum less at most SLACK (-inf: nothing yet)
   double s;   // sum exp(x - m)
   double u;   // sum exp(x - m) (x - m)
-  float my;   // running maximum of y
+  float my;   // reference of y
   double sy;  // sum exp(y - my)
   double w;   // sum exp(x - m) ((x - m) - (y - my))
 };
@@ -105,40 +113,19 @@ __device__ __forceinline__ void rebase_y(Acc& a, float M) {
   a.my = M;
 }
 
-__device__ __forceinline__ void merge(Acc& a, Acc b, bool kl) {
-  const float M = fmaxf(a.m, b.m);
-  rebase_x(a, M);
-  rebase_x(b, M);
-  if (kl) {
-    const float My = fmaxf(a.my, b.my);
-    rebase_y(a, My);
-    rebase_y(b, My);
-    a.sy += b.sy;
-    a.w += b.w;
-  }
-  a.s += b.s;
-  a.u += b.u;
-}
-
-__device__ __forceinline__ Acc shfl_acc(const Acc& a, int src) {
-  Acc r;
-  r.m = __shfl(a.m, src, WAVE);
-  r.s = __shfl(a.s, src, WAVE);
-  r.u = __shfl(a.u, src, WAVE);
-  r.my = __shfl(a.my, src, WAVE);
-  r.sy = __shfl(a.sy, src, WAVE);
-  r.w = __shfl(a.w, src, WAVE);
-  return r;
-}
-
 }  // namespace
 
-template <class D, bool KL>
+template <class D, bool KL, int NT_RS>
 __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) {
   using C = RowChunk<D>;
   constexpr int N = C::N;
-  constexpr int U_RS = 4;  // chunks per thread in flight (8 lowers the occupancy and the bandwidth)
+  constexpr int NW_RS = NT_RS / WAVE;
+  // chunks per thread in flight: with 4 the 16-bit instantiations hold too
+  // many registers for the waves that keep HBM busy (4096 bf16 rows of V =
+  // 128256: 188 us at 4, 174 us at 2, 6.0 TB/s; with KL, 2048 rows: 218 / 214 us)
+  constexpr int U_RS = 2;
   __shared__ Acc part[NW_RS];
+  __shared__ float ref_m[NW_RS], ref_my[NW_RS];
   const int tid = threadIdx.x;
   const int64_t r = blockIdx.x;
   const int V = static_cast<int>(a.vocab);
@@ -172,8 +159,7 @@ __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) 
         for (int e = 0; e < N; ++e) xs[k][e] = ys[k][e] = -__builtin_inff();
       }
     }
-    // maxima of the iteration's chunks first: at most one re-base per
-    // iteration (padding is -inf)
+    // maxima of the iteration's chunks first (padding is -inf)
     float cm = xs[0][0], cmy = ys[0][0];
 #pragma unroll
     for (int k = 0; k < U_RS; ++k)
@@ -182,10 +168,10 @@ __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) 
         cm = fmaxf(cm, xs[k][e]);
         if (KL) cmy = fmaxf(cmy, ys[k][e]);
       }
-    if (cm > acc.m) rebase_x(acc, cm);
-    if (KL && cmy > acc.my) rebase_y(acc, cmy);
+    if (cm > acc.m + SLACK) rebase_x(acc, cm);
+    if (KL && cmy > acc.my + SLACK) rebase_y(acc, cmy);
     // exponents in base 2: d2 = (x - m) log2(e) in one rounding; the base-2
-    // sums of the iteration (at most U_RS * N terms, each at most 1) are
+    // sums of the iteration (at most U_RS * N terms, each below e^SLACK) are
     // scaled to natural units and added to the float64 partials once
     const float mb = acc.m * LOG2E_F, myb = acc.my * LOG2E_F;
     float fs = 0.0f, fu = 0.0f, fsy = 0.0f, fw = 0.0f;
@@ -235,18 +221,42 @@ __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) 
       acc.w += static_cast<double>(fw) * LN2_D;
     }
   }
-  // merge: wave tree, then the waves in order
-#pragma unroll
-  for (int off = WAVE / 2; off > 0; off >>= 1) {
-    const Acc o = shfl_acc(acc, (tid & (WAVE - 1)) ^ off);
-    merge(acc, o, KL);
+  // merge: the row's largest references first, so that each thread re-bases
+  // its partial once (two double-precision exponentials), then plain sums in a
+  // fixed tree.  (Merging partial by partial re-based twice per step of the
+  // tree: 4096 bf16 rows of V = 4099 took 38.0 us, now 28.6.)
+  const int wave = tid / WAVE;
+  const float wm = wave_reduce(acc.m, OpMax()), wmy = KL ? wave_reduce(acc.my, OpMax()) : 0.0f;
+  if ((tid & (WAVE - 1)) == 0) {
+    ref_m[wave] = wm;
+    ref_my[wave] = wmy;
   }
-  if ((tid & (WAVE - 1)) == 0) part[tid / WAVE] = acc;
+  __syncthreads();
+  float M = ref_m[0], My = ref_my[0];
+#pragma unroll
+  for (int i = 1; i < NW_RS; ++i) {
+    M = fmaxf(M, ref_m[i]);
+    My = fmaxf(My, ref_my[i]);
+  }
+  rebase_x(acc, M);
+  if (KL) rebase_y(acc, My);  // (from the thread's own s: before the sums)
+  acc.s = wave_reduce(acc.s, OpAdd());
+  acc.u = wave_reduce(acc.u, OpAdd());
+  if (KL) {
+    acc.sy = wave_reduce(acc.sy, OpAdd());
+    acc.w = wave_reduce(acc.w, OpAdd());
+  }
+  if ((tid & (WAVE - 1)) == 0) part[wave] = acc;
   __syncthreads();
   if (tid != 0) return;
   Acc t = part[0];
 #pragma unroll
-  for (int i = 1; i < NW_RS; ++i) merge(t, part[i], KL);
+  for (int i = 1; i < NW_RS; ++i) {
+    t.s += part[i].s;
+    t.u += part[i].u;
+    t.sy += part[i].sy;
+    t.w += part[i].w;
+  }
   const double logS = log(t.s);
   if (a.out_entropy) a.out_entropy[r] = static_cast<float>(logS - t.u / t.s);
   if (a.out_lse) a.out_lse[r] = static_cast<float>(static_cast<double>(t.m) + logS);
@@ -261,19 +271,28 @@ __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) 
   }
 }
 
+// Threads per row: 256 where rows are many (their merges overlap other rows'
+// reads); 1024 where a CU gets one row at most, so that the row has 16 waves'
+// loads in flight instead of 4.  f32 with KL, V = 50257: 255 rows 34.2 us with
+// 256 threads, 22.2 us with 1024; 520 rows 41.4 against 47.9 us.
+constexpr int64_t RS_FEW_ROWS = 256;
+
 hipError_t launch_row_stats(const fl_row_stats_args& a, hipStream_t s) {
-  const dim3 grid(static_cast<unsigned>(a.rows)), block(NT_RS);
-  const bool kl = a.ref_logits != nullptr;
-  if (a.dtype == FL_DTYPE_F32) {
-    if (kl) hipLaunchKernelGGL((k_row_stats<F32, true>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((k_row_stats<F32, false>), grid, block, 0, s, a);
-  } else if (a.dtype == FL_DTYPE_BF16) {
-    if (kl) hipLaunchKernelGGL((k_row_stats<BF16, true>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((k_row_stats<BF16, false>), grid, block, 0, s, a);
-  } else {
-    if (kl) hipLaunchKernelGGL((k_row_stats<F16, true>), grid, block, 0, s, a);
-    else hipLaunchKernelGGL((k_row_stats<F16, false>), grid, block, 0, s, a);
-  }
+  const dim3 grid(static_cast<unsigned>(a.rows));
+  const bool few = a.rows <= RS_FEW_ROWS;
+  auto run = [&](auto d) {
+    using D = decltype(d);
+    auto go = [&](auto kl_c) {
+      constexpr bool KL = decltype(kl_c)::value;
+      if (few) hipLaunchKernelGGL((k_row_stats<D, KL, 1024>), grid, dim3(1024), 0, s, a);
+      else hipLaunchKernelGGL((k_row_stats<D, KL, 256>), grid, dim3(256), 0, s, a);
+    };
+    if (a.ref_logits != nullptr) go(std::true_type{});
+    else go(std::false_type{});
+  };
+  if (a.dtype == FL_DTYPE_F32) run(F32{});
+  else if (a.dtype == FL_DTYPE_BF16) run(BF16{});
+  else run(F16{});
   return hipGetLastError();
 }
 

@@ -1,0 +1,59 @@
+"""Row statistics at the edges of the work-group split and of the reference
+that a thread's sums are relative to (MI355X), against float64."""
+
+import pytest
+import torch
+
+from rl_project_amd import row_stats
+
+pytestmark = pytest.mark.gpu
+
+
+def _check(x, y, lab, tol):
+    out = row_stats(x, lab, y, entropy=True, lse=True)
+    a = torch.log_softmax(x.double(), -1)
+    want = {"logprob": a.gather(-1, lab[:, None])[:, 0], "entropy": -(a.exp() * a).sum(-1),
+            "kl": (a.exp() * (a - torch.log_softmax(y.double(), -1))).sum(-1), "lse": torch.logsumexp(x.double(), -1)}
+    for name, w in want.items():
+        got = getattr(out, name).double()
+        assert torch.allclose(got, w, rtol=tol, atol=tol * (1.0 + float(w.abs().max()))), (name, float((got - w).abs().max()))
+
+
+# one row per CU and more (256 / 257 rows: 1024 / 256 threads a row); rows shorter
+# than an iteration, its edges, and several iterations
+@pytest.mark.parametrize("R", [1, 256, 257])
+@pytest.mark.parametrize("V", [1, 7, 2047, 2048, 2049, 4096, 8193, 16385])
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+def test_rows_and_lengths(R, V, dt):
+    print(f"[rowstats shapes R={R} V={V} {dt}]", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(R + V)
+    x = (3.0 * torch.randn(R, V, generator=g, device="cuda")).to(dt)
+    y = (3.0 * torch.randn(R, V, generator=g, device="cuda")).to(dt)
+    # (float sums of at most 16 terms in float64 partials: a few 2^-24)
+    _check(x, y, torch.randint(0, V, (R,), generator=g, device="cuda"), 1e-6)
+
+
+@pytest.mark.parametrize("order", ["rising", "falling", "late peak", "far apart"])
+@pytest.mark.parametrize("R", [3, 300])
+def test_references_that_move(order, R):
+    """Values that pass a thread's reference again and again, once, or by less
+    than it takes to move it; and rows whose threads hold references far apart."""
+    print(f"[rowstats references {order} R={R}]", flush=True)
+    V = 40000
+    g = torch.Generator(device="cuda").manual_seed(R)
+    x = torch.randn(R, V, generator=g, device="cuda")
+    y = torch.randn(R, V, generator=g, device="cuda")
+    ramp = torch.linspace(-60.0, 60.0, V, device="cuda")
+    if order == "rising":
+        x, y = x + ramp, y + 0.5 * ramp
+    elif order == "falling":
+        x, y = x - ramp, y + ramp
+    elif order == "late peak":
+        x[:, -1] = 7.5     # (within the slack of most references)
+        x[:, -2000] = 30.0
+        y[:, 5] = 50.0
+    else:
+        x[:, ::7] -= 300.0
+        y[:, 1::3] -= 80.0
+    # (the scores reach 100: a float term's exponent is rounded to 2^-24 of that)
+    _check(x, y, torch.randint(0, V, (R,), generator=g, device="cuda"), 2e-5)
