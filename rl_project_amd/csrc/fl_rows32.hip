@@ -108,7 +108,7 @@ struct Shared32 {
       uint64_t mass[NB];
     };
     struct {
-      uint64_t acc[NBF + 1];  // two-read bins: packed sums, then exclusive mass prefixes; [NBF]: discard slot
+      uint64_t acc[NBF];   // two-read bins: packed sums, then exclusive mass prefixes
       uint32_t pc[NBF];    // exclusive count prefixes
     };
     alignas(16) uint32_t tkc[1 << 13];  // top-k path bins (key >> 19)
@@ -643,9 +643,13 @@ __device__ __forceinline__ uint32_t topk_count4(Shared32& sh, const Xform& X, in
   if (4 * ch + 3 < V) {
     bad |= sm != sm;
 #pragma unroll
-    for (int e = 0; e < 4; ++e) {
-      k[e] = f32_key(s[e]);
-      atomicAdd(&sh.tkc[k[e] >> TK_SH], 1u);
+    for (int e = 0; e < 4; ++e) k[e] = f32_key(s[e]);
+    // (a chunk of -inf alone, as in a masked vocabulary, is not counted: its
+    // adds would queue at one LDS counter, and a K-th value at -inf declines
+    // the row whatever that count is)
+    if (max(max(k[0], k[1]), max(k[2], k[3])) > KEY_NEG_INF) {
+#pragma unroll
+      for (int e = 0; e < 4; ++e) atomicAdd(&sh.tkc[k[e] >> TK_SH], 1u);
     }
   } else {
 #pragma unroll
@@ -1071,7 +1075,10 @@ __device__ __forceinline__ bool read1(Shared32& sh, const Src& S, const Xform& X
   if (!(ka > KEY_NEG_INF && ka < KEY_POS_INF && fabsf(A) < 1048576.0f)) return false;
   c = A + ANCHOR_UP;
 
-  // branch-free: an element outside the bins adds 0 to the discard slot
+  // One element: a value of -inf (a masked vocabulary, a filtered row) or above
+  // the bins adds nothing -- neither is kept, weighted or decided on here -- as
+  // all such adds would queue at one LDS counter (softmax sampling of a row of
+  // V = 50257 with 50 finite values: 69.0 us, now 34.9).
   auto add = [&](int idx, float y) __attribute__((always_inline)) {
     const bool valid = idx < V;
     bad |= (valid && y != y) ? 2u : 0u;
@@ -1079,10 +1086,11 @@ __device__ __forceinline__ bool read1(Shared32& sh, const Src& S, const Xform& X
     const bool ok = valid && y <= c;
     km = max(km, ok ? f32_key(y) : 0u);
     nfin += (ok && y > -__builtin_inff()) ? 1u : 0u;
-    const int b = fbin(y, c);
-    const uint64_t w = (1ull << CNT_SH) | fterm(y, c);
-    atomicAdd(reinterpret_cast<unsigned long long*>(&sh.acc[ok ? b : NBF]),
-              static_cast<unsigned long long>(ok ? w : 0ull));
+    if (ok && y > -__builtin_inff()) {
+      const int b = fbin(y, c);
+      const uint64_t w = (1ull << CNT_SH) | fterm(y, c);
+      atomicAdd(reinterpret_cast<unsigned long long*>(&sh.acc[b]), static_cast<unsigned long long>(w));
+    }
   };
   // A chunk of 4 whose values are all valid, finite and inside the bins (the
   // usual case) needs no per-element test: its maximum, minimum and sum
@@ -1101,6 +1109,8 @@ __device__ __forceinline__ bool read1(Shared32& sh, const Src& S, const Xform& X
         const uint64_t w = (1ull << CNT_SH) | fterm(y[e], c);
         atomicAdd(reinterpret_cast<unsigned long long*>(&sh.acc[b]), static_cast<unsigned long long>(w));
       }
+    } else if (4 * ch + 3 < V && mx == -__builtin_inff() && sm == sm) {
+      km = max(km, KEY_NEG_INF);  // (a chunk of -inf alone)
     } else {
 #pragma unroll
       for (int e = 0; e < 4; ++e) add(4 * ch + e, y[e]);
