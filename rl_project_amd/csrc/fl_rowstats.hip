@@ -33,14 +33,15 @@ namespace fl {
 namespace {
 
 constexpr float LOG2E_F = 1.44269504088896340736f;
-constexpr double LN2_D = 0.69314718055994530942;
+constexpr double INV_LOG2E_F = 1.0 / static_cast<double>(LOG2E_F);  // (of the float: a base-2 difference over it is exact)
 // A thread moves its reference m only once a value passes it by more than
 // this: a re-base is a double-precision exponential, and while every new
 // maximum took one, some lane of a wave had one in nearly every iteration
-// (4096 bf16 rows of V = 128256: 195 us, without it 188 us).  Terms stay below
-// e^8, far from any float's range, and every sum is relative to m whatever
-// m is.
-constexpr float SLACK = 8.0f;
+// (4096 bf16 rows of V = 128256: 195 us, without it 188 us).  The terms that
+// count have exponents up to SLACK log2(e): below 8 they round at 2^-22 like
+// those a little under the maximum (a slack of 8 is 1 % faster, but 255 bf16
+// rows of V = 50257 are then 6.2e-7 from the KL in 64 bits, with 5.5 2.7e-7).
+constexpr float SLACK = 5.5f;
 
 template <class D>
 struct RowChunk;
@@ -87,6 +88,17 @@ struct Acc {
   double w;   // sum exp(x - m) ((x - m) - (y - my))
 };
 
+// The reference a partial's terms were taken against.  Exponents are
+// fma(x, log2(e), -mb) with mb = RN(m log2(e)), so that is mb / log2(e) and
+// not m: half an ulp of mb is up to 3e-7 of every term of the thread.  (255
+// f32 rows of V = 50257 with KL, from 64 bits: 3.5e-7 with m, 3.2e-7 with
+// mb / log2(e); entropies of scores around 12: 6.4e-8 and 2.6e-8.)  Where mb overflows (a mask of the type's lowest value) the
+// exponents are (x - m) log2(e).
+__device__ __forceinline__ bool base2_ok(float m) { return __builtin_fabsf(m * LOG2E_F) != __builtin_inff(); }
+__device__ __forceinline__ double ref_of(float m) {
+  return base2_ok(m) ? static_cast<double>(m * LOG2E_F) * INV_LOG2E_F : static_cast<double>(m);
+}
+
 // Re-base a partial on a larger maximum M (m <= M).  A partial with no
 // element yet (m == -inf) has zero sums and stays zero.
 __device__ __forceinline__ void rebase_x(Acc& a, float M) {
@@ -94,7 +106,7 @@ __device__ __forceinline__ void rebase_x(Acc& a, float M) {
     a.m = M;
     return;
   }
-  const double d = static_cast<double>(a.m) - static_cast<double>(M);
+  const double d = ref_of(a.m) - ref_of(M);
   const double f = exp(d);
   a.u = (a.u + a.s * d) * f;
   a.w = (a.w + a.s * d) * f;
@@ -106,7 +118,7 @@ __device__ __forceinline__ void rebase_y(Acc& a, float M) {
     a.my = M;
     return;
   }
-  const double d = static_cast<double>(a.my) - static_cast<double>(M);
+  const double d = ref_of(a.my) - ref_of(M);
   // (x - m) - (y - M) = (x - m) - (y - my) - d
   a.w -= a.s * d;
   a.sy *= exp(d);
@@ -175,8 +187,8 @@ __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) 
     // scaled to natural units and added to the float64 partials once
     const float mb = acc.m * LOG2E_F, myb = acc.my * LOG2E_F;
     float fs = 0.0f, fu = 0.0f, fsy = 0.0f, fw = 0.0f;
-    const bool finite_max = acc.m != -__builtin_inff() && (!KL || acc.my != -__builtin_inff());
-    if (c0 + (U_RS - 1) * NT_RS + tid < nfull && finite_max) {
+    const bool bx = base2_ok(acc.m), by = !KL || base2_ok(acc.my);
+    if (c0 + (U_RS - 1) * NT_RS + tid < nfull && bx && by) {
       // whole chunks under a finite maximum: -inf gives d2 = -inf, e = 0 and
       // e * d2 = NaN, the reference's 0 * -inf
 #pragma unroll
@@ -194,20 +206,24 @@ __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) 
           }
         }
     } else {
-      // the row's last chunks (partial or past the row) and values before any
-      // finite one (-inf below a maximum that is still -inf)
+      // the row's last chunks (partial or past the row), values before any
+      // finite one (-inf below a maximum that is still -inf) and references
+      // whose base-2 form overflows
+      auto below = [](float x, float m, float b, bool ok) {
+        return x == -__builtin_inff() ? x : ok ? fmaf(x, LOG2E_F, -b) : (x - m) * LOG2E_F;
+      };
 #pragma unroll
       for (int k = 0; k < U_RS; ++k) {
         const int c = c0 + k * NT_RS + tid;
 #pragma unroll
         for (int e = 0; e < N; ++e) {
           if (N * c + e >= V) continue;
-          const float d2 = xs[k][e] == -__builtin_inff() ? -__builtin_inff() : fmaf(xs[k][e], LOG2E_F, -mb);
+          const float d2 = below(xs[k][e], acc.m, mb, bx);
           const float ex = __builtin_amdgcn_exp2f(d2);
           fs += ex;
           fu += ex * d2;
           if (KL) {
-            const float dy2 = ys[k][e] == -__builtin_inff() ? -__builtin_inff() : fmaf(ys[k][e], LOG2E_F, -myb);
+            const float dy2 = below(ys[k][e], acc.my, myb, by);
             fsy += __builtin_amdgcn_exp2f(dy2);
             fw += ex * (d2 - dy2);
           }
@@ -215,10 +231,10 @@ __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) 
       }
     }
     acc.s += fs;
-    acc.u += static_cast<double>(fu) * LN2_D;
+    acc.u += static_cast<double>(fu) * INV_LOG2E_F;
     if (KL) {
       acc.sy += fsy;
-      acc.w += static_cast<double>(fw) * LN2_D;
+      acc.w += static_cast<double>(fw) * INV_LOG2E_F;
     }
   }
   // merge: the row's largest references first, so that each thread re-bases
@@ -259,14 +275,14 @@ __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) 
   }
   const double logS = log(t.s);
   if (a.out_entropy) a.out_entropy[r] = static_cast<float>(logS - t.u / t.s);
-  if (a.out_lse) a.out_lse[r] = static_cast<float>(static_cast<double>(t.m) + logS);
+  if (a.out_lse) a.out_lse[r] = static_cast<float>(ref_of(t.m) + logS);
   if (KL && a.out_kl) a.out_kl[r] = static_cast<float>(t.w / t.s - logS + log(t.sy));
   if (a.labels && a.out_logprob) {
     const int64_t lab = a.labels[r];
     float lp;
     if (lab == a.ignore_index) lp = -0.0f;  // -(cross_entropy = 0) for an ignored target
     else if (lab < 0 || lab >= V) lp = __builtin_nanf("");
-    else lp = static_cast<float>(static_cast<double>(C::elem(rx, static_cast<int>(lab))) - static_cast<double>(t.m) - logS);
+    else lp = static_cast<float>(static_cast<double>(C::elem(rx, static_cast<int>(lab))) - ref_of(t.m) - logS);
     a.out_logprob[r] = lp;
   }
 }

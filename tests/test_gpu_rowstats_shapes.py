@@ -57,3 +57,36 @@ def test_references_that_move(order, R):
         y[:, 1::3] -= 80.0
     # (the scores reach 100: a float term's exponent is rounded to 2^-24 of that)
     _check(x, y, torch.randint(0, V, (R,), generator=g, device="cuda"), 2e-5)
+
+
+@pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
+@pytest.mark.parametrize("R", [3, 300])
+@pytest.mark.parametrize("masked", [5000, 20000])
+def test_rows_that_begin_with_the_lowest_value(dt, R, masked):
+    """A mask of the type's lowest value (its base-2 exponent overflows) over a
+    row's head, so that threads begin with it, and over the whole row."""
+    print(f"[rowstats lowest {dt} R={R} masked={masked}]", flush=True)
+    V = 20000
+    g = torch.Generator(device="cuda").manual_seed(R)
+    x = torch.randn(R, V, generator=g, device="cuda").to(dt)
+    x[:, :masked] = torch.finfo(dt).min
+    lab = torch.randint(min(masked, V - 100), V, (R,), generator=g, device="cuda")
+    out = row_stats(x, lab, entropy=False, lse=True)
+    a = torch.log_softmax(x.double(), -1).gather(-1, lab[:, None])[:, 0]
+    assert torch.allclose(out.logprob.double(), a, rtol=1e-6, atol=1e-6)
+    assert torch.allclose(out.lse.double(), torch.logsumexp(x.double(), -1), rtol=1e-6, atol=1e-6)
+
+
+@pytest.mark.parametrize("R", [255, 600])
+@pytest.mark.parametrize("V", [512, 4099, 50257])
+def test_entropy_is_as_good_as_its_own_rounding(R, V):
+    """Scores around 12: the rounding of a reference's base-2 form, up to 3e-7,
+    would be in every term of its thread.  Bound: a float32 result's own
+    rounding, 2^-24 of it."""
+    print(f"[rowstats entropy R={R} V={V}]", flush=True)
+    g = torch.Generator(device="cuda").manual_seed(R + V)
+    x = 2.5 * torch.randn(R, V, generator=g, device="cuda") + 12.0
+    out = row_stats(x, torch.zeros(R, dtype=torch.int64, device="cuda"), entropy=True)
+    a = torch.log_softmax(x.double(), -1)
+    want = -(a.exp() * a).sum(-1)
+    assert float((out.entropy.double() - want).norm() / want.norm()) < 2.0 ** -24
