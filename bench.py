@@ -430,7 +430,7 @@ def bench_lmhead(args, dev) -> int:
         "roofline": _roofline(alg_bytes, step_ms, args.workload, step_ms_mean=step_ms,
                               isolated_step_ms_p10=durs[len(durs) // 10],
                               isolated_step_ms_p90=durs[(9 * len(durs)) // 10],
-                              kernel="k_lm_prep + k_lm_sample + k_lm_thresh + k_lm_gemm + k_lm_pick",
+                              kernel="k_lm_sample + k_lm_thresh + k_lm_gemm + k_lm_pick",
                               mfma_tflops=flops / (step_ms * 1e-3) / 1e12, mfma_peak_tflops=2500.0),
         "unfused": {"ms_per_step": unf_ms, "matmul_ms": gemm_ms,
                     "note": "torch.matmul(h, W.T) into [B, V] bf16 logits, then fl_sample (SamplerPlan)"},

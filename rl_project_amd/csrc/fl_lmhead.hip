@@ -2,14 +2,15 @@
 // logits, lm_head(h[:, -1, :]) at transformer/model.py:190 and :201, sampled
 // by generation/sampling.py:16-61), for rows that all use top-k.
 //
-//   prep    one work-group per row: the row's history bitmap (one bit per
-//           vocabulary id, which also de-duplicates the ids) and counters;
 //   sample  a gemm over every S-th vocabulary row (ns <= 8192 rows,
 //           S = ceil(vocab / 8192)), in tiles of 64 rows so that many work-groups
-//           share the work; it stores each sampled value's order key.  A
-//           logit's value does not depend on its kernel: the same MFMA chain
-//           over the same dim order produces it in both gemms;
-//   thresh  one work-group per row: the k-th largest sampled key.  The sampled
+//           share the work; it stores each sampled logit.  A logit's value does
+//           not depend on its kernel: the same MFMA chain over the same dim
+//           order produces it in both gemms.  Beside it in the launch, one
+//           work-group per row: the row's history bitmap (one bit per
+//           vocabulary id, which also de-duplicates the ids) and counters;
+//   thresh  one work-group per row: the k-th largest sampled key (soft-cap,
+//           penalty and temperature applied here).  The sampled
 //           values are a subset of the row's, so at least k of the row's values
 //           reach it: a lower bound of the row's k-th largest value;
 //   gemm    logits = hidden · weightᵀ on the matrix cores
@@ -40,6 +41,7 @@ typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 typedef float floatx4 __attribute__((ext_vector_type(4)));
 
 constexpr int LM_NT = 256;                 // threads of the gemm and pick work-groups
+constexpr int LM_NTT = 1024;               // threads of the thresh work-groups (one 16-byte piece of sampled logits each)
 constexpr int LM_NTILE = 256;              // vocabulary rows per gemm tile
 constexpr int LM_GW = 8;                   // waves per main-gemm work-group (32 vocabulary rows each)
 constexpr int LM_GSLOTS = 2;               // main-gemm stages in flight (register slots)
@@ -101,13 +103,13 @@ struct LmWs {
   uint32_t* cnt;    // [batch, LM_CNT_LD] candidates appended (word 0 of a row's 256 bytes)
   uint32_t* stat;   // [batch] FL_ROW_* bits found by prep and gemm
   uint32_t* bits;   // [batch, bw] history bitmap
-  uint16_t* skey;   // [batch, nsl] keys of the sampled rows (entry e: vocabulary row e·S)
+  uint16_t* skey;   // [batch, nsl] bf16 patterns of the sampled logits (entry e: vocabulary row e·S)
   uint64_t* cand;   // [batch, LM_CAP] (key << 32) | ~vocabulary index
   int bw;           // words per bitmap row, a multiple of 4
   int stride;       // S
   int ns;
   int nsl;          // ns rounded up to a multiple of 8
-  int prep;         // the call passes a penalty: the prep kernel runs and sets stat
+  int prep;         // the call passes a penalty: the rows' histories are prepared, which sets stat
 };
 
 __host__ __device__ inline int lm_stride(int64_t vocab) {  // ceil(vocab / 8192): ns <= 8192
@@ -206,14 +208,17 @@ __device__ uint32_t wave_kth_key(int n, int k, uint32_t* hist, KeyAt&& key_at) {
 }  // namespace
 
 // ---------------------------------------------------------------- prep
-// Launched when the call passes a penalty and histories; one work-group per
-// row.  A penalised row gets its history bitmap (one bit per vocabulary id,
-// which also de-duplicates the ids), built in LDS and written out whole;
-// every row gets its status from its history (too long, ids out of range).
-__global__ __launch_bounds__(LM_NT) void k_lm_prep(const fl_lm_head_args a, LmWs ws) {
-  __shared__ __attribute__((aligned(16))) uint32_t sbits[FL_MAX_VOCAB_16 / 32];   // (bw <= this)
+// A penalised row gets its history bitmap (one bit per vocabulary id, which
+// also de-duplicates the ids), built in LDS and written out whole; every row
+// gets its status from its history (too long, ids out of range).  One
+// work-group per row, in the sample gemm's launch when the call passes a
+// penalty and histories: that gemm leaves half the CUs idle, and nothing in it
+// needs the bitmaps (a launch of its own took 5 us).
+namespace {
+// sbits: ws.bw (a multiple of 4) words of LDS, 16-byte aligned
+__device__ void lm_prep_row(const fl_lm_head_args& a, const LmWs& ws, int b, uint32_t* sbits) {
   __shared__ uint32_t s_flags;
-  const int b = blockIdx.x, tid = threadIdx.x;
+  const int tid = threadIdx.x;
   const bool pen = row_penalised(a, b);
   if (tid == 0) s_flags = 0u;
   int H = pen ? a.hist_len[b] : 0;
@@ -244,54 +249,28 @@ __global__ __launch_bounds__(LM_NT) void k_lm_prep(const fl_lm_head_args a, LmWs
   }
   if (tid == 0) ws.stat[b] = s_flags;
 }
-
-// ---------------------------------------------------------------- row parameters
-// The sample gemm's rows' parameters in LDS, filled once per work-group
-// (thread m loads row m's before the gemm's loop, into registers, and stores
-// them to LDS after it), so its epilogue computes every key without a memory
-// round trip.
-template <int MR>
-struct LmRows {
-  float T[MR], RT[MR], RP[MR];   // temperature, RN(1 / T) (0 for greedy), penalty (1: none)
-  uint32_t pen[MR];              // the row is penalised
-};
-struct LmRowReg {
-  float T, RP;
-  uint32_t pen;
-};
-__device__ __forceinline__ LmRowReg lm_row_load(const fl_lm_head_args& a, int m) {
-  LmRowReg r{1.0f, 1.0f, 0u};
-  if (m < a.batch) {
-    r.T = a.temperature[m];
-    r.pen = row_penalised(a, m) ? 1u : 0u;
-    r.RP = r.pen ? a.repetition_penalty[m] : 1.0f;
-  }
-  return r;
-}
-template <int MR>
-__device__ __forceinline__ void lm_row_store(LmRows<MR>& p, int m, const LmRowReg& r) {
-  p.T[m] = r.T;
-  p.RT[m] = r.T > 0.0f ? recip_rt(r.T) : 0.0f;
-  p.RP[m] = r.RP;
-  p.pen[m] = r.pen;
-}
+}  // namespace
 
 // ---------------------------------------------------------------- sample gemm
 // The sampled rows: vocabulary rows e·S for tile entries e, 16 per wave and 64
-// per work-group (ns / 64 work-groups), the keys of their transformed values
-// stored to ws.skey.  MB: 16-row blocks of the batch (1, 2 or 4).  Each
+// per work-group (ns / 64 work-groups), their logits' bf16 patterns stored to
+// ws.skey (the thresh kernel transforms them).  Work-groups past those prepare
+// the rows' histories.  MB: 16-row blocks of the batch (1, 2 or 4).  Each
 // 16 x 16 block of logits is one wave's MFMA chain over the dim in 32-wide
 // steps in ascending order, as in the main gemm below, so a sampled value
 // equals the main gemm's value of the same logit bit for bit.
 template <int MB>
 __global__ __launch_bounds__(LM_NT) void k_lm_sample(const fl_lm_head_args a, LmWs ws) {
   constexpr int NST = 8;                            // register slots (stages in flight)
-  constexpr int MR = 16 * MB;
   constexpr int NE = 16 * (LM_NT / WAVE);          // sampled entries per work-group
-  constexpr int BP = MR * NE / LM_NT;              // history words per thread
-  __shared__ __attribute__((aligned(16))) uint16_t sA[2][16 * MB * LM_AST];
-  __shared__ LmRows<MR> sRows;
-  __shared__ uint32_t sBits[MR][NE];                // word of entry j's vocabulary row in row m's bitmap
+  constexpr int STAGES_B = 2 * 16 * MB * LM_AST * 2, BITS_B = FL_MAX_VOCAB_16 / 8;   // (4 bw <= BITS_B)
+  __shared__ __attribute__((aligned(16))) unsigned char lds[STAGES_B > BITS_B ? STAGES_B : BITS_B];
+  const int gemm_groups = (ws.ns + NE - 1) / NE;
+  if (static_cast<int>(blockIdx.x) >= gemm_groups) {
+    lm_prep_row(a, ws, static_cast<int>(blockIdx.x) - gemm_groups, reinterpret_cast<uint32_t*>(lds));
+    return;
+  }
+  uint16_t (*sA)[16 * MB * LM_AST] = reinterpret_cast<uint16_t (*)[16 * MB * LM_AST]>(lds);
   const int tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid >> 6;
   const int B = static_cast<int>(a.batch), D = static_cast<int>(a.dim);
   const int S = ws.stride, ns = ws.ns;
@@ -346,17 +325,6 @@ __global__ __launch_bounds__(LM_NT) void k_lm_sample(const fl_lm_head_args a, Lm
     }
   };
 
-  // the rows' parameters and, for a penalty, the history words of the
-  // tile's sampled rows, loaded now and put into LDS after the loop
-  const LmRowReg rowp = lm_row_load(a, tid);
-  uint32_t bitp[BP];
-#pragma unroll
-  for (int q = 0; q < BP; ++q) {
-    const int i = tid + LM_NT * q, m = i / NE, j = i % NE;
-    const int e = min(e0 + j, ns - 1);
-    bitp[q] = (ws.prep && m < B) ? ws.bits[static_cast<size_t>(m) * ws.bw + ((e * S) >> 5)] : 0u;
-  }
-
   // Pipeline: stage s (its weight fragments and its hidden pieces) lives in
   // register slot s % NST.  Iteration `it` stores the hidden pieces of stage
   // it + 1 into LDS buffer (it + 1) & 1, multiplies stage it, and refills its
@@ -388,35 +356,13 @@ __global__ __launch_bounds__(LM_NT) void k_lm_sample(const fl_lm_head_args a, Lm
       __syncthreads();
     }
   }
-  if (tid < MR) lm_row_store(sRows, tid, rowp);
-#pragma unroll
-  for (int q = 0; q < BP; ++q) {
-    const int i = tid + LM_NT * q;
-    sBits[i / NE][i % NE] = bitp[q];
-  }
-  __syncthreads();
-  // the sampled values' keys: bf16 rounding (the logit), then soft-cap,
-  // penalty and temperature (lm_tval, as the thresholds and the pick apply them)
-  const float cap = a.softcap;
-  const int n = eme * S;
-  uint32_t key[MB][4];
+  // the sampled logits (bf16 rounding)
 #pragma unroll
   for (int mb = 0; mb < MB; ++mb) {
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int m = 16 * mb + 4 * l4 + r;
-      const bool ok = m < B && eme < ns;
-      const bool member = ok && sRows.pen[m] != 0u && ((sBits[m][16 * w + l16] >> (n & 31)) & 1u);
-      const float y = lm_tval(BF16::from_f32(acc[mb][0][r]), cap, member, sRows.RP[m], sRows.T[m], sRows.RT[m]);
-      key[mb][r] = ok ? lm_key_of(y) : 0u;
-    }
-  }
-#pragma unroll
-  for (int mb = 0; mb < MB; ++mb) {
-#pragma unroll
-    for (int r = 0; r < 4; ++r) {
-      const int m = 16 * mb + 4 * l4 + r;
-      if (m < B && eme < ns) ws.skey[static_cast<size_t>(m) * ws.nsl + eme] = static_cast<uint16_t>(key[mb][r]);
+      if (m < B && eme < ns) ws.skey[static_cast<size_t>(m) * ws.nsl + eme] = static_cast<uint16_t>(BF16::from_f32(acc[mb][0][r]));
     }
   }
 }
@@ -672,9 +618,12 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(NW / 
 // ---------------------------------------------------------------- thresh
 // The row's bound, then its raw-key thresholds, and the row's counters.
 // The bound is the K-th largest of the row's sampled keys (none when fewer
-// than K were sampled): the keys go into LDS in 16-byte pieces, then two
-// passes of a 256-bin histogram (high byte, then the low byte within the
-// chosen high byte), every wave counting into a histogram of its own.
+// than K were sampled).  A thread reads one 16-byte piece of the sampled logits
+// and keeps its eight transformed keys in registers for two passes of a
+// histogram in LDS: the upper 12 bits, then the lower 4 within the chosen bin.
+// (With 8 + 8 bits, nearly all of a row's keys fell into some ten bins of the
+// first pass and their atomics queued, 64x4096x128256: 9.8 us, now 9.3 with
+// the transforms that the sample gemm did before.)
 // Soft-cap, penalty and temperature are monotone (non-decreasing) in the
 // logit, separately for history members and the rest, so "transformed key
 // >= bound" is "raw key >= a threshold" for each class; wave 0 finds the
@@ -682,73 +631,83 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(NW / 
 // over the keys of the non-NaN bf16 patterns.  A penalty that is not a
 // positive finite number breaks the monotony: such a row reports
 // FL_ROW_LIMIT.
-__global__ __launch_bounds__(LM_NT) void k_lm_thresh(const fl_lm_head_args a, LmWs ws) {
-  constexpr int NW = LM_NT / WAVE;
-  __shared__ uint4 keys[LM_NSAMPLE / 8];
-  __shared__ uint32_t hist[NW][256];
+__global__ __launch_bounds__(LM_NTT) void k_lm_thresh(const fl_lm_head_args a, LmWs ws) {
+  constexpr int NW = LM_NTT / WAVE;
+  static_assert(NW == 16 && LM_NTT * 8 >= LM_NSAMPLE, "4096 bins: 256 per wave; one piece per thread");
+  __shared__ uint4 hist4[4096 / 4];
+  __shared__ uint32_t low[16], s_tot[NW];
   __shared__ int s_bin;
   __shared__ uint32_t s_above;
+  uint32_t* hist = reinterpret_cast<uint32_t*>(hist4);
   const int b = blockIdx.x, tid = threadIdx.x, lane = tid & (WAVE - 1), w = tid >> 6;
   if (tid == 0) {
     ws.cnt[b * LM_CNT_LD] = 0u;
     if (!ws.prep) ws.stat[b] = 0u;
+    s_bin = -1;
   }
   const int K = a.top_k[b];
   const bool topk = K >= 1 && K <= FL_LM_HEAD_MAX_TOPK;   // (else the pick reports the row)
+  const float T = a.temperature[b], RT = T > 0.0f ? recip_rt(T) : 0.0f, cap = a.softcap;
+  const bool pen = row_penalised(a, b);
+  const float RP = pen ? a.repetition_penalty[b] : 1.0f;
   uint32_t bound = 0;   // transformed key; 0: none
   if (topk) {
-    const int ns = ws.ns, nq = (ns + 7) >> 3;
-    const uint4* src = reinterpret_cast<const uint4*>(ws.skey + static_cast<size_t>(b) * ws.nsl);
-    for (int i = tid; i < nq; i += LM_NT) keys[i] = src[i];
-    int k = K;
-    uint32_t prefix = 0;   // high byte, once chosen
-    for (int pass = 0; pass < 2; ++pass) {
-      for (int i = tid; i < NW * 256; i += LM_NT) (&hist[0][0])[i] = 0u;
-      __syncthreads();   // (pass 0: also the keys)
-      for (int i = tid; i < nq; i += LM_NT) {
-        const uint4 q = keys[i];
-        const uint32_t wd[4] = {q.x, q.y, q.z, q.w};
-        const int nj = min(8, ns - 8 * i);
+    hist4[tid] = make_uint4(0u, 0u, 0u, 0u);
+    if (tid < 16) low[tid] = 0u;
+    const int ns = ws.ns, nj = ns - 8 * tid;   // keys of this thread (8 or more: 8)
+    uint32_t key[8];
+    if (nj > 0) {
+      const uint4 q = reinterpret_cast<const uint4*>(ws.skey + static_cast<size_t>(b) * ws.nsl)[tid];
+      const uint32_t wd[4] = {q.x, q.y, q.z, q.w};
+      const uint32_t* hb = ws.bits + static_cast<size_t>(b) * ws.bw;
+      uint32_t hw[8];
 #pragma unroll
-        for (int j = 0; j < 8; ++j) {
-          const uint32_t key = (wd[j >> 1] >> (16 * (j & 1))) & 0xFFFFu;
-          if (j < nj) {
-            if (pass == 0) atomicAdd(&hist[w][key >> 8], 1u);
-            else if ((key >> 8) == prefix) atomicAdd(&hist[w][key & 0xFFu], 1u);
-          }
-        }
+      for (int j = 0; j < 8; ++j) hw[j] = pen ? hb[(min(8 * tid + j, ns - 1) * ws.stride) >> 5] : 0u;
+#pragma unroll
+      for (int j = 0; j < 8; ++j) {
+        const int n = min(8 * tid + j, ns - 1) * ws.stride;
+        const uint32_t bits = (wd[j >> 1] >> (16 * (j & 1))) & 0xFFFFu;
+        key[j] = lm_key_of(lm_tval(bits, cap, (hw[j] >> (n & 31)) & 1u, RP, T, RT));
       }
-      __syncthreads();
-      if (w == 0) {
-        uint32_t c4[4], above = 0;
+    }
+    __syncthreads();
 #pragma unroll
-        for (int q = 0; q < 4; ++q) {
-          uint32_t c = 0;
+    for (int j = 0; j < 8; ++j)
+      if (j < nj) atomicAdd(&hist[key[j] >> 4], 1u);
+    __syncthreads();
+    // wave w holds the 256 bins below 4096 - 256 w
+    uint32_t c4[4], above = 0;
 #pragma unroll
-          for (int v = 0; v < NW; ++v) c += hist[v][255 - 4 * lane - q];
-          c4[q] = c;
-        }
-        const int bin = wave_top_bin(c4, k, above);
-        if (lane == 0) {
-          s_bin = bin;
-          s_above = above;
-        }
+    for (int q = 0; q < 4; ++q) c4[q] = hist[4095 - 256 * w - 4 * lane - q];
+    const uint32_t tot = wave_reduce(c4[0] + c4[1] + c4[2] + c4[3], OpAdd());
+    if (lane == 0) s_tot[w] = tot;
+    __syncthreads();
+    uint32_t higher = 0;
+    for (int v = 0; v < w; ++v) higher += s_tot[v];
+    const uint32_t k = static_cast<uint32_t>(K);
+    if (higher < k && higher + tot >= k) {
+      const int bin = wave_top_bin(c4, static_cast<int>(k - higher), above);
+      if (lane == 0) {
+        s_bin = 3840 - 256 * w + bin;
+        s_above = higher + above;
       }
+    }
+    __syncthreads();
+    const int bin = s_bin;
+    if (bin >= 0) {   // (else fewer than K keys: no bound)
+#pragma unroll
+      for (int j = 0; j < 8; ++j)
+        if (j < nj && static_cast<int>(key[j] >> 4) == bin) atomicAdd(&low[key[j] & 15u], 1u);
       __syncthreads();
-      const int bin = s_bin;
-      if (bin < 0) break;   // fewer than K keys: no bound
-      k -= static_cast<int>(s_above);
-      if (pass == 0) prefix = static_cast<uint32_t>(bin);
-      else bound = (prefix << 8) | static_cast<uint32_t>(bin);
+      const uint32_t incl = wave_incl_scan(lane < 16 ? low[15 - lane] : 0u);
+      const uint64_t m = __ballot(incl + s_above >= k);
+      bound = (static_cast<uint32_t>(bin) << 4) | static_cast<uint32_t>(16 - __ffsll(static_cast<unsigned long long>(m)));
     }
   }
   // wave v finds threshold v: candidates of non-members, of members, +inf
   // of non-members, of members (a row without a penalty has no members)
   static_assert(NW >= 4, "one wave per threshold");
   if (w >= 4) return;
-  const float T = a.temperature[b], RT = T > 0.0f ? recip_rt(T) : 0.0f, cap = a.softcap;
-  const bool pen = row_penalised(a, b);
-  const float RP = pen ? a.repetition_penalty[b] : 1.0f;
   const bool bad = pen && !(RP > 0.0f && RP <= 3.402823466e38f);
   if (w == 0 && bad && lane == 0) atomicOr(&ws.stat[b], static_cast<uint32_t>(FL_ROW_LIMIT));
   const bool member = pen && (w & 1), inf = w >= 2;
@@ -996,14 +955,13 @@ hipError_t launch_lm_head(const fl_lm_head_args& a, hipStream_t s) {
   LmWs ws = lm_ws(a.workspace, a.batch, a.vocab);
   ws.prep = a.repetition_penalty != nullptr && a.hist_ids != nullptr && a.hist_len != nullptr;
   const dim3 rows(static_cast<unsigned>(a.batch));
-  if (ws.prep) hipLaunchKernelGGL(k_lm_prep, rows, dim3(LM_NT), 0, s, a, ws);
-  const dim3 stiles(static_cast<unsigned>((ws.ns + 63) / 64));
+  const dim3 stiles(static_cast<unsigned>((ws.ns + 63) / 64 + (ws.prep ? a.batch : 0)));
   const dim3 tiles(static_cast<unsigned>((a.vocab + 255) / 256));
   const int mb = static_cast<int>((a.batch + 15) / 16);
   auto run = [&](auto tag_mb) {
     constexpr int MB = decltype(tag_mb)::value;
     hipLaunchKernelGGL((k_lm_sample<MB>), stiles, dim3(LM_NT), 0, s, a, ws);
-    hipLaunchKernelGGL(k_lm_thresh, rows, dim3(LM_NT), 0, s, a, ws);
+    hipLaunchKernelGGL(k_lm_thresh, rows, dim3(LM_NTT), 0, s, a, ws);
     hipLaunchKernelGGL((k_lm_gemm<MB, LM_GW>), tiles, dim3(LM_GW * WAVE), 0, s, a, ws);
   };
   if (mb <= 1) run(std::integral_constant<int, 1>{});

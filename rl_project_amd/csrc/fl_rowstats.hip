@@ -40,7 +40,7 @@ constexpr double INV_LOG2E_F = 1.0 / static_cast<double>(LOG2E_F);  // (of the f
 // (4096 bf16 rows of V = 128256: 195 us, without it 188 us).  The terms that
 // count have exponents up to SLACK log2(e): below 8 they round at 2^-22 like
 // those a little under the maximum (a slack of 8 is 1 % faster, but 255 bf16
-// rows of V = 50257 are then 6.2e-7 from the KL in 64 bits, with 5.5 2.7e-7).
+// rows of V = 50257 are then 6.2e-7 from the KL in 64 bits, with 5.5 3.3e-7).
 constexpr float SLACK = 5.5f;
 
 template <class D>
