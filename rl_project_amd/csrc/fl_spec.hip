@@ -44,6 +44,7 @@ struct Chunk;
 template <>
 struct Chunk<F32> {
   static constexpr int N = 4;
+  __device__ static float at(const char* row, int64_t i) { return reinterpret_cast<const float*>(row)[i]; }
   __device__ static float elem(__amdgpu_buffer_rsrc_t r, int i) {
     return __uint_as_float(__builtin_amdgcn_raw_buffer_load_b32(r, 4 * i, 0, 0));
   }
@@ -57,6 +58,7 @@ struct Chunk<F32> {
 template <class H>
 struct Chunk16 {
   static constexpr int N = 8;
+  __device__ static float at(const char* row, int64_t i) { return H::to_f32(reinterpret_cast<const uint16_t*>(row)[i]); }
   __device__ static float elem(__amdgpu_buffer_rsrc_t r, int i) {
     return H::to_f32(__builtin_amdgcn_raw_buffer_load_b16(r, 2 * i, 0, 0));
   }
@@ -110,8 +112,11 @@ struct SharedSpec {
 // in the logits' dtype (:63), accept iff u_accept < ratio (:65).  Writes the
 // ratios and the accepted drafts when `write`; returns the accepted count,
 // *rej = whether a draft was rejected.
+// (Inlined, with write_tail below: a call takes the address of the kernel's
+// arguments, which then live in scratch memory, and every pointer in them is
+// a flat one.)
 template <class D>
-__device__ int accept_walk(const fl_spec_args& a, int64_t b, bool* rej, bool write = true) {
+__device__ __forceinline__ int accept_walk(const fl_spec_args& a, int64_t b, bool* rej, bool write = true) {
   // Called by one whole wave: lane l evaluates positions l, l + 64, ... in
   // parallel (their loads in flight together); the first position whose
   // draw fails the ratio ends the walk, as the sequential rule has it.
@@ -124,23 +129,25 @@ __device__ int accept_walk(const fl_spec_args& a, int64_t b, bool* rej, bool wri
   int64_t n = K;  // accepted drafts (the first rejected position, if any)
   for (int64_t i0 = 0; i0 < K && n == K; i0 += WAVE) {
     const int64_t i = i0 + lane;
-    float ratio = 0.0f;
+    float ratio = 0.0f, u = 1.0f;
     int64_t d = -1;
     bool acc = false;
     if (i < K) {
       d = a.draft_ids[b * K + i];
+      u = a.u_accept[b * K + i];
       if (d >= 0 && d < V) {
         const fl_row_desc td = a.target_desc[b * (K + 1) + i];
         const fl_row_desc dd = a.draft_desc[b * K + i];
         const char* tp = static_cast<const char*>(a.target) + (b * (K + 1) + i) * a.ld * esz;
         const char* dp = static_cast<const char*>(a.draft) + (b * K + i) * a.ld * esz;
-        const __amdgpu_buffer_rsrc_t rt = row_rsrc(tp, static_cast<uint32_t>(V * esz));
-        const __amdgpu_buffer_rsrc_t rd = row_rsrc(dp, static_cast<uint32_t>(V * esz));
-        const float p = prob_of<D>(td, filt_value<D>(C::elem(rt, static_cast<int>(d)), a.softcap, T), d);
-        const float q = prob_of<D>(dd, filt_value<D>(C::elem(rd, static_cast<int>(d)), a.softcap, T), d);
+        // (global loads: every lane has rows of its own, and a buffer resource
+        // per lane becomes a loop over the lanes, one memory round trip each)
+        const float xt = C::at(tp, d), xd = C::at(dp, d);
+        const float p = prob_of<D>(td, filt_value<D>(xt, a.softcap, T), d);
+        const float q = prob_of<D>(dd, filt_value<D>(xd, a.softcap, T), d);
         ratio = fminf(1.0f, D::rn(p / D::rn(q + 1e-10f)));
       }
-      acc = a.u_accept[b * K + i] < ratio;
+      acc = u < ratio;
     }
     const uint64_t fail = __ballot(i < K && !acc);
     const int64_t f = fail ? i0 + __ffsll(static_cast<unsigned long long>(fail)) - 1 : K;
@@ -166,7 +173,13 @@ struct PairRows {
   fl_row_desc td, dd;
   int V, nch, nfull;
   float cap, T;
-  __device__ PairRows(const fl_spec_args& a, int64_t b, int pos) {
+  // (readfirstlane: the position comes through memory, so the compiler takes
+  // it for one that differs by lane, and a buffer resource that does is a
+  // loop over the lanes around every load with a full wait after it: the
+  // first slice pass, 6 sequences of bf16 V = 50257: 13.2 us, so 7.5; 32 of
+  // f32 V = 128256: 21.4, so 17.9, of it 3.5 from the walk's loads above)
+  __device__ __forceinline__ PairRows(const fl_spec_args& a, int64_t b, int lane_pos) {
+    const int pos = __builtin_amdgcn_readfirstlane(lane_pos);
     const int64_t K = a.k;
     const size_t esz = D::id == FL_DTYPE_F32 ? 4 : 2;
     V = static_cast<int>(a.vocab);
@@ -183,7 +196,9 @@ struct PairRows {
   }
   // the raw logits of chunk c of both rows
   __device__ __forceinline__ void load(int c, float (&xt)[N], float (&xd)[N]) const {
-    if (c < nfull) {
+    // (float32 dwords past the row read zeros; the last value of an odd 16-bit
+    // row shares its dword with one past it and is read by itself)
+    if (D::id == FL_DTYPE_F32 || c < nfull) {
       C::unpack(buf_load16(rt, 16u * c, 0u), xt);
       C::unpack(buf_load16(rd, 16u * c, 0u), xd);
     } else {
