@@ -22,7 +22,7 @@
 //   entropy      = log S - u / S
 //   KL           = w / S - log S + log S'
 // A -inf logit contributes exp(-inf) * (-inf) = NaN to u and w, as 0 * -inf
-// does in the reference's expression.
+// does in the reference's expression; a finite one, however low, does not.
 #include <type_traits>
 
 #include "fl_device.h"
@@ -187,8 +187,10 @@ __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) 
     // scaled to natural units and added to the float64 partials once
     const float mb = acc.m * LOG2E_F, myb = acc.my * LOG2E_F;
     float fs = 0.0f, fu = 0.0f, fsy = 0.0f, fw = 0.0f;
+    double wd = 0.0;
     const bool bx = base2_ok(acc.m), by = !KL || base2_ok(acc.my);
-    if (c0 + (U_RS - 1) * NT_RS + tid < nfull && bx && by) {
+    bool general = !(c0 + (U_RS - 1) * NT_RS + tid < nfull && bx && by);
+    if (!general) {
       // whole chunks under a finite maximum: -inf gives d2 = -inf, e = 0 and
       // e * d2 = NaN, the reference's 0 * -inf
 #pragma unroll
@@ -205,27 +207,45 @@ __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) 
             fw = fmaf(ex, d2 - dy2, fw);
           }
         }
-    } else {
+    }
+    // A finite value near the type's lowest (a mask) has d2 = -inf too, where
+    // the reference's 0 * x is 0 (and p * -y large, but finite): such an
+    // iteration is taken again below.  Not once a -inf logit has made the
+    // wave's sum NaN, and the row's with it, so that a row with many of them
+    // takes one such iteration a wave.
+    const bool nan_u = !(__builtin_fabsf(fu) < __builtin_inff());
+    const bool nan_w = KL && !(__builtin_fabsf(fw) < __builtin_inff());
+    if (__any(nan_u || nan_w)) {
+      const bool lost_u = __any(acc.u != acc.u), lost_w = KL && __any(acc.w != acc.w);
+      general = general || (nan_u && !lost_u) || (nan_w && !lost_w);
+    }
+    if (general) {
       // the row's last chunks (partial or past the row), values before any
-      // finite one (-inf below a maximum that is still -inf) and references
-      // whose base-2 form overflows
+      // finite one (-inf below a maximum that is still -inf), references whose
+      // base-2 form overflows, and values whose exponent does
       auto below = [](float x, float m, float b, bool ok) {
         return x == -__builtin_inff() ? x : ok ? fmaf(x, LOG2E_F, -b) : (x - m) * LOG2E_F;
       };
+      // (the difference itself, also where it is past the float range)
+      auto wide = [](float d2, float x, float m) -> double {
+        return d2 == -__builtin_inff() && x != d2 ? (static_cast<double>(x) - ref_of(m)) * LOG2E_F : d2;
+      };
+      fs = fu = fsy = 0.0f;
+      fw = 0.0f;
 #pragma unroll
       for (int k = 0; k < U_RS; ++k) {
         const int c = c0 + k * NT_RS + tid;
 #pragma unroll
         for (int e = 0; e < N; ++e) {
           if (N * c + e >= V) continue;
-          const float d2 = below(xs[k][e], acc.m, mb, bx);
+          const float x = xs[k][e], d2 = below(x, acc.m, mb, bx);
           const float ex = __builtin_amdgcn_exp2f(d2);
           fs += ex;
-          fu += ex * d2;
+          fu += d2 == -__builtin_inff() && x != d2 ? 0.0f : ex * d2;
           if (KL) {
-            const float dy2 = below(ys[k][e], acc.my, myb, by);
+            const float y = ys[k][e], dy2 = below(y, acc.my, myb, by);
             fsy += __builtin_amdgcn_exp2f(dy2);
-            fw += ex * (d2 - dy2);
+            wd += static_cast<double>(ex) * (wide(d2, x, acc.m) - wide(dy2, y, acc.my));
           }
         }
       }
@@ -234,7 +254,7 @@ __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) 
     acc.u += static_cast<double>(fu) * INV_LOG2E_F;
     if (KL) {
       acc.sy += fsy;
-      acc.w += static_cast<double>(fw) * INV_LOG2E_F;
+      acc.w += (static_cast<double>(fw) + wd) * INV_LOG2E_F;
     }
   }
   // merge: the row's largest references first, so that each thread re-bases
