@@ -599,7 +599,7 @@ struct RowOut {
 //            histogram on bits 31..TK_SH of its order-preserving key (16 bins
 //            per binade); the row's first 4 * TK_TILE * NT keys stay in
 //            registers
-//   history  each element of the history bitmap moves from the bin of s to
+//   history  each id of the history, counted once, moves from the bin of s to
 //            the bin of z = penalty(s)
 //   scan     the bin of the K-th largest z (a descending block scan)
 //   read 2   every element in that bin or above becomes a candidate
@@ -737,7 +737,10 @@ __device__ __forceinline__ void topk_hist_move(Shared32& sh, const Src& S, const
     bad |= z != z;
     const uint32_t ks = f32_key(s), kz = f32_key(z);
     if ((ks >> TK_SH) != (kz >> TK_SH)) {
-      atomicSub(&sh.tkc[ks >> TK_SH], 1u);
+      // (the bin of -inf may not have counted it, see topk_count4, and below
+      // zero it would reach the scan's NaN bits: a penalty below 0 moves such
+      // an element to +inf)
+      if (ks > KEY_NEG_INF) atomicSub(&sh.tkc[ks >> TK_SH], 1u);
       atomicAdd(&sh.tkc[kz >> TK_SH], 1u);
     }
     return kz;
@@ -893,8 +896,9 @@ __device__ __forceinline__ bool topk_path(Shared32& sh, const Src& S, const Xfor
     uint32_t sum = 0;
 #pragma unroll
     for (int q = 0; q < TK_BPT; ++q) sum += c[q];
-    // (the scan also counts the threads that saw a NaN, in bits 20 and up:
-    // a row holds at most 2^18 values and a block 1024 threads)
+    // (the scan also counts the threads that saw a NaN, in bits 20 and up: a
+    // row holds at most 2^18 values, its history adds at most 2^16 to the
+    // bins, and a block has 1024 threads)
     uint32_t tot;
     const uint32_t ex = block_excl_scan<uint32_t>(sum | (bad ? 1u << 20 : 0u), sh.redu, &tot) & 0xFFFFFu;
     // (with a NaN no bin is picked: pick_bin stays -1 and the two-read path

@@ -56,3 +56,20 @@ def test_masked_row_statuses():
         out = sample_tokens(x.cuda(), temperature=0.8, top_k=K, uniforms=torch.full((4,), 0.5).cuda(), check_status=False)
         assert out.status.tolist() == [16, 1, 2, 0], K
         assert out.tokens.tolist() == [-1, -1, -1, 9000]
+
+
+@pytest.mark.parametrize("rp", [-1.0, 1.3])
+@pytest.mark.parametrize("at", [0, 4 * 1022, 50000])
+def test_masked_history_and_a_nan(at, rp):
+    """History ids on -inf logits, whose chunks are not counted, do not hide a
+    NaN of the row under any penalty (one below 0 makes them +inf): the status
+    of a top-k row is that of the same row without top-k."""
+    print(f"[rows32 masked history NaN at={at} rp={rp}]", flush=True)
+    V = 50257
+    x = torch.full((2, V), float("-inf"))
+    x[:, 100:200] = torch.randn(2, 100, generator=torch.Generator().manual_seed(at))
+    x[1, at] = float("nan")
+    hist = torch.arange(30000, 30010, dtype=torch.int32).repeat(2, 1).cuda()
+    got = [sample_tokens(x.cuda(), temperature=0.8, top_k=K, repetition_penalty=rp, history=hist,
+                         uniforms=torch.full((2,), 0.5).cuda(), check_status=False).status.tolist() for K in (0, 1, 50)]
+    assert got[0][1] & 1 and got[1] == got[0] and got[2] == got[0], got
