@@ -88,8 +88,10 @@ def row_stats(logits: torch.Tensor, labels: Optional[torch.Tensor] = None, ref_l
     # A label out of range gives a NaN log-probability (and is never read
     # through), so the labels are looked at only where some row has one: a sum
     # in place of the five launches of the test itself, ahead of the kernel.
-    # (log-probabilities are at most 0, so a sum is NaN only through a NaN)
-    if lab is not None and check_labels and R > 0 and math.isnan(o_lp.sum().item()):
+    # (log-probabilities are at most 0, so a sum is NaN only through a NaN; an
+    # ignore_index past the vocabulary is refused as a label, yet ignored by
+    # the kernel)
+    if lab is not None and check_labels and R > 0 and (ignore_index >= V or math.isnan(o_lp.sum().item())):
         bad = ((lab < 0) & (lab != ignore_index)) | (lab >= V)
         if bool(bad.any()):
             raise IndexError(f"target {int(lab[bad][0])} is out of bounds for {V} classes")

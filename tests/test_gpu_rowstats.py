@@ -108,3 +108,14 @@ def test_random_row_stats_cases():
         assert _close(st.entropy, L.entropy_from_logits(x), 2e-5)[0], seed
         assert _close(st.kl, L.kl_full_distribution(x, y), 2e-5)[0], seed
         assert _close(st.lse, L.logsumexp(x), 2e-5, 1e-6)[0], seed
+
+
+def test_ignore_index_past_the_vocabulary_is_no_label():
+    """A label past the vocabulary is refused also where ``ignore_index`` names
+    it; without one such an ignore_index changes nothing."""
+    x = torch.randn(4, 100).cuda()
+    for index in (100, 1000):
+        with pytest.raises(IndexError):
+            row_stats(x, torch.tensor([3, index, 1, 2]).cuda(), ignore_index=index)
+        assert torch.equal(row_stats(x, torch.tensor([3, 99, 1, 2]).cuda(), ignore_index=index).logprob,
+                           row_stats(x, torch.tensor([3, 99, 1, 2]).cuda()).logprob)
