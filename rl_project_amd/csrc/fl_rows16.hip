@@ -50,6 +50,12 @@ constexpr int LOOKAHEAD = FL_LOOKAHEAD;          // row chunks per thread in fli
 static_assert(LOOKAHEAD >= EARLY_CHUNKS && LOOKAHEAD <= NCH, "lookahead window");
 constexpr int SHORT_MAX = 512;                   // entries one wave decides over
 constexpr int XSLOTS = 4;                        // slots past the tile in flight
+// A row of at most one chunk per thread goes chunk by chunk: through the tile
+// it also pays for 15 slots that hold nothing.  64 bf16 rows, per launch, tile /
+// without: V = 513 18.6 / 15.4 us, 4099 20.3 / 17.7, 8192 20.8 / 18.4; from two
+// chunks per thread on the tile's loads in flight win (V = 12001 odd starts:
+// 21.1 us with it, 22.9 without).
+constexpr int ONE_CHUNK_V = NT * 8;
 constexpr int MAX_HEAVY = 8;                     // patterns with more than 65535 values (at most 5 exist)
 
 static_assert(NSLOT * NT * 8 == FL_MAX_VOCAB_16 && NSLOT >= NCH, "identification slots cover the longest row");
@@ -149,8 +155,8 @@ __device__ __forceinline__ ScanHit scan_first(Shared16& sh, int n, bool total_gi
 // 16-byte chunk c (elements 8c .. 8c+7) of a row; elements >= V read as 0.
 // (A row of an odd vocabulary starts at any multiple of 2 bytes; neither global
 // nor buffer loads of 16 bytes need more alignment than that, so every row
-// takes them and the register tile: 30 bf16 rows of V = 50257, which used to
-// go element by element, 43.3 -> 27.9 us per launch.)
+// takes them, and the register tile from two chunks per thread on: 30 bf16 rows
+// of V = 50257, which used to go element by element, 43.3 -> 27.9 us per launch.)
 typedef uint32_t u32x4_a2 __attribute__((ext_vector_type(4), aligned(2)));
 __device__ __forceinline__ uint4 load_chunk16(const uint16_t* row, int c, int V) {
   const int e0 = c * 8;
@@ -351,8 +357,8 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
   const bool SC_ELEM = SC && SC_ELEM_IN;
   const int nfull = V >> 3;                               // chunks holding 8 valid elements
   // the row (as far as it reaches) through the VGPR tile, values past the tile
-  // streamed
-  const bool fast_row = !HEAVY && !SC_ELEM && nfull > 0;
+  // streamed; a row of at most one chunk per thread without the tile
+  const bool fast_row = !HEAVY && !SC_ELEM && V > ONE_CHUNK_V;
   const int nslots = WIDE ? (((V + 7) >> 3) + NT - 1) / NT : NCH;  // slots of NT chunks
 
   // ------------------------------------------------ loads
