@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from rl_project_amd import filtered_outputs, sample_tokens, workloads
-from tests.helpers import classify_workload, unpack_mask
+from tests.helpers import classify_workload, unfiltered_values, unpack_mask
 
 pytestmark = pytest.mark.gpu
 
@@ -87,3 +87,22 @@ def test_status_of_short_lists():
     ok = sample_tokens(x[3:].to(torch.bfloat16).cuda(), temperature=0.9, top_k=20, top_p=0.9,
                        uniforms=torch.full((2,), 0.3).cuda())
     assert ok.status.tolist() == [0, 0] and int(ok.tokens[1]) == int(out.tokens[4])
+
+
+@pytest.mark.parametrize("K", [1, 64, 300, 513])
+def test_soft_capped_top_k_lists(K):
+    print(f"[rows16 short softcap K={K}]", flush=True)
+    w = _rows(K, 6, 20000, torch.bfloat16)
+    T = w.temperature.clone()
+    T[4] = 0.0
+    w = dataclasses.replace(w, temperature=T, softcap=30.0, top_k=torch.full((6,), K, dtype=torch.int32),
+                            repetition_penalty=torch.tensor([1.0, 1.2, 1.0, 1.2, 1.0, 1.0]))
+    wd = w.to("cuda")
+    out = sample_tokens(wd.logits, return_logprobs=True, **wd.kwargs())
+    kw = wd.kwargs()
+    kw.pop("uniforms")
+    filt, _, mask, status = filtered_outputs(wd.logits, want_mask=True, **kw)
+    assert int(status.abs().sum()) == 0
+    summ, verdicts = classify_workload(w, out.tokens, unpack_mask(mask, w.vocab), got_values=filt.cpu(),
+                                       got_all_values=unfiltered_values(wd.logits, kw).cpu())
+    assert all(v.ok for v in verdicts), (summ, [v.details for v in verdicts if not v.ok][:2])

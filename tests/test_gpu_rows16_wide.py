@@ -7,7 +7,7 @@ import pytest
 import torch
 
 from rl_project_amd import filtered_outputs, sample_tokens, workloads
-from tests.helpers import classify_workload, unpack_mask
+from tests.helpers import classify_workload, unfiltered_values, unpack_mask
 
 pytestmark = pytest.mark.gpu
 
@@ -38,4 +38,34 @@ def test_past_the_tile(V, kind):
     assert int(status.abs().sum()) == 0
     assert int(out.tokens[3]) == V - 1
     summ, verdicts = classify_workload(w, out.tokens, unpack_mask(mask, V))
+    assert all(v.ok for v in verdicts), (summ, [v.details for v in verdicts if not v.ok][:2])
+
+
+@pytest.mark.parametrize("V", [131073, 139271, 262143])
+@pytest.mark.parametrize("zero_top", [False, True])
+def test_soft_capped_rows_past_the_tile(V, zero_top):
+    """Soft-capped rows without a history, which take the streamed slots too
+    (and read their tile again): the odd last value certain, and +0.0, the
+    padding's pattern, the largest."""
+    print(f"[rows16 wide softcap V={V} zero_top={zero_top}]", flush=True)
+    B, dt = 3, torch.float16 if zero_top else torch.bfloat16
+    w = workloads.make("hetero_bf16_256x128256", seed=V, batch=B, vocab=V)
+    x = w.logits.float()
+    if zero_top:
+        x = -torch.round(x.abs() * 4.0) / 4.0 + 0.0
+        x[0, : V - 3] -= 1.0
+    else:
+        x[2, V - 1] = 60.0
+    w = dataclasses.replace(w, logits=x.to(dt), softcap=30.0, repetition_penalty=torch.ones(B),
+                            temperature=torch.tensor([1.0, 0.7, 0.2]), top_k=torch.tensor([0, 50, 0], dtype=torch.int32))
+    wd = w.to("cuda")
+    out = sample_tokens(wd.logits, return_logprobs=True, **wd.kwargs())
+    kw = wd.kwargs()
+    kw.pop("uniforms")
+    filt, _, mask, status = filtered_outputs(wd.logits, want_mask=True, **kw)
+    assert int(status.abs().sum()) == 0
+    if not zero_top:
+        assert int(out.tokens[2]) == V - 1
+    summ, verdicts = classify_workload(w, out.tokens, unpack_mask(mask, V), got_values=filt.cpu(),
+                                       got_all_values=unfiltered_values(wd.logits, kw).cpu())
     assert all(v.ok for v in verdicts), (summ, [v.details for v in verdicts if not v.ok][:2])
