@@ -48,7 +48,16 @@ constexpr int EARLY_CHUNKS = 4;                  // row chunks per thread reques
 #endif
 constexpr int LOOKAHEAD = FL_LOOKAHEAD;          // row chunks per thread in flight while counting
 static_assert(LOOKAHEAD >= EARLY_CHUNKS && LOOKAHEAD <= NCH, "lookahead window");
-constexpr int SHORT_MAX = 512;                   // entries one wave decides over
+// Entries one wave decides over: its rounds of 64 against the block phases'
+// barriers and scans.  SHORT_MAX where the row has more entries than threads
+// (64 f16 rows of V = 8192 with 2000 entries under top-k 512: 17.4 us, block
+// phases 17.6; under top-k 256 16.4 / 17.5).  With fewer, where a thread of the
+// block phases has one entry, SHORT_CUT under top-p or min-p and SHORT_PLAIN for
+// a draw (or maximum) alone.  64 f16 rows of V = 512, one wave / block: top-p 0.9
+// with 300 entries 15.3 / 16.0 us, 450 16.6 / 16.6; top-p 0.99 with 300 16.2 /
+// 16.0, 450 17.7 / 16.6; the draw alone with 128 13.5 / 14.1, 192 14.5 / 14.6,
+// 256 15.3 / 14.8, 500 18.4 / 15.3.
+constexpr int SHORT_MAX = 512, SHORT_CUT = 384, SHORT_PLAIN = 192;
 constexpr int XSLOTS = 4;                        // slots past the tile in flight
 // A row of at most one chunk per thread goes chunk by chunk: through the tile
 // it also pays for 15 slots that hold nothing.  64 bf16 rows, per launch, tile /
@@ -844,8 +853,8 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
   // ---------------- short lists: one wave decides
   // Every decision of a top-k row (a request's default keeps 50) acts on the
   // entries down to its K-th value, at most K and the run equal to it, and a
-  // short row has few entries to begin with.  For up to SHORT_MAX of them, wave
-  // 0 takes all the decisions with wave scans, in the arithmetic of the block
+  // short row has few entries to begin with.  For a short list of them, wave 0
+  // takes all the decisions with wave scans, in the arithmetic of the block
   // phases below (integer sums: the same results bit for bit), while the other
   // waves sum the counts of all entries for the total's check.  The phases of
   // a long list are chains of block barriers and two dozen LDS round trips:
@@ -854,7 +863,8 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
   bool done = false;
   if constexpr (!HEAVY) {
     const bool tk = K > 0 && K < V;
-    if (N > 0 && (N <= SHORT_MAX || (tk && K <= SHORT_MAX))) {  // block-uniform
+    const int most = N > NT ? SHORT_MAX : (TP > 0.0f && TP < 1.0f) || MP > 0.0f ? SHORT_CUT : SHORT_PLAIN;
+    if (N > 0 && (N <= most || (tk && K <= SHORT_MAX))) {  // block-uniform
       if (tid < WAVE) {
         float* const Ys = reinterpret_cast<float*>(sh.hist + SLICE_BASE);
         float* const Es = Ys + SHORT_MAX;
@@ -881,7 +891,7 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
             }
           }
         }
-        if (n <= SHORT_MAX) {
+        if (n <= most) {
           // values, weights and exclusive prefixes
           uint32_t rc = 0;
           uint64_t rm = 0;

@@ -106,3 +106,23 @@ def test_soft_capped_top_k_lists(K):
     summ, verdicts = classify_workload(w, out.tokens, unpack_mask(mask, w.vocab), got_values=filt.cpu(),
                                        got_all_values=unfiltered_values(wd.logits, kw).cpu())
     assert all(v.ok for v in verdicts), (summ, [v.details for v in verdicts if not v.ok][:2])
+
+
+# (the longest lists of a wave: 192 entries for the draw alone, 384 under top-p
+# or min-p, 512 of a row with more entries than threads)
+@pytest.mark.parametrize("n", [191, 192, 193, 383, 384, 385, 511, 512, 513, 1023, 1024, 1025])
+@pytest.mark.parametrize("K", [0, 150, 300, 512])
+def test_edges_of_the_wave_s_lists(n, K):
+    """Rows of n distinct values, several of each, under every kind of cut."""
+    print(f"[rows16 short n={n} K={K}]", flush=True)
+    V = 3 * n + 1
+    w = _rows(n, 6, V, torch.float16)
+    vals = (torch.linspace(-8.0, 8.0, 2 * n + 2).to(torch.float16).unique())[:n]
+    assert vals.numel() == n
+    g = torch.Generator().manual_seed(n + K)
+    x = vals[torch.stack([torch.randperm(V, generator=g) % n for _ in range(6)])]
+    _check(dataclasses.replace(w, logits=x, top_k=torch.full((6,), K, dtype=torch.int32),
+                               temperature=torch.tensor([1.0, 0.7, 2.0, 0.0, 1.3, 0.0]),
+                               top_p=torch.tensor([1.0, 0.9, 1.0, 1.0, 0.99, 0.9]),
+                               min_p=torch.tensor([0.0, 0.0, 0.02, 0.0, 0.0, 0.02]),
+                               repetition_penalty=torch.ones(6)))
