@@ -298,9 +298,10 @@ struct OpMax { template <typename T> __device__ T operator()(T a, T b) const { r
 
 // Wave-level reduction / scan through rocPRIM's cross-lane (DPP) primitives;
 // the combination order is fixed, so floating-point results are deterministic.
-template <typename T, class Op>
+// (W lanes: the wave's, or each of its aligned groups of W)
+template <typename T, class Op, int W = WAVE>
 __device__ __forceinline__ T wave_reduce(T v, Op op) {
-  using WR = rocprim::warp_reduce<T, WAVE, true>;
+  using WR = rocprim::warp_reduce<T, W, true>;
   typename WR::storage_type st;
   T out;
   WR().reduce(v, out, st, op);

@@ -10,19 +10,23 @@
 // One work-group per row; the row streams through 16-byte chunks interleaved
 // over the threads (coalesced), 2 chunks per thread in flight.  The loads need
 // no more than an element's alignment, so rows of an odd vocabulary take them
-// too (4096 bf16 rows of V = 50257: element by element 309 us, so 132 us).  Each thread keeps, relative to a reference m
+// too (4096 bf16 rows of V = 50257: element by element 309 us, so 86 us).  HBM
+// bounds it from some hundred rows on: 4096 bf16 rows of V = 128256 171 us, 6.1
+// TB/s.  Each thread keeps, relative to a reference m
 // near its maximum of the row x,
 //   s = sum exp(x - m),  u = sum exp(x - m) (x - m),
 // and with a reference row y (its m') also
 //   s' = sum exp(y - m'),  w = sum exp(x - m) ((x - m) - (y - m')),
 // in float64, rescaled when m moves.  The partials are added in a fixed tree
-// once all are relative to the row's largest m, so results are deterministic.
+// once all are relative to the largest m, the same for every call: a row's
+// results are a function of the row alone.
 // With M that reference and S the row's sum:
 //   log p(label) = x_label - M - log S
 //   entropy      = log S - u / S
 //   KL           = w / S - log S + log S'
 // A -inf logit contributes exp(-inf) * (-inf) = NaN to u and w, as 0 * -inf
 // does in the reference's expression; a finite one, however low, does not.
+#include <algorithm>
 #include <type_traits>
 
 #include "fl_device.h"
@@ -38,10 +42,15 @@ constexpr double INV_LOG2E_F = 1.0 / static_cast<double>(LOG2E_F);  // (of the f
 // this: a re-base is a double-precision exponential, and while every new
 // maximum took one, some lane of a wave had one in nearly every iteration
 // (4096 bf16 rows of V = 128256: 195 us, without it 188 us).  The terms that
-// count have exponents up to SLACK log2(e): below 8 they round at 2^-22 like
-// those a little under the maximum (a slack of 8 is 1 % faster, but 255 bf16
-// rows of V = 50257 are then 6.2e-7 from the KL in 64 bits, with 5.5 3.3e-7).
-constexpr float SLACK = 5.5f;
+// count have exponents up to SLACK log2(e), rounded at that size: of the KL's
+// distance from 64 bits, summed over 72 sets of rows each of f32, bf16 and f16,
+// 3.5 gives 2.29e-5, 3.14e-5 and 3.28e-5, 5.5 2.38e-5, 3.36e-5 and 3.46e-5 (and
+// 162 us in place of 171 for the 4096 rows).  The same for both rows: their differences are
+// what counts, and with 1 for the reference row alone the KL is 4.5e-5 off.
+constexpr float SLACK = 3.5f;
+// Stands for the values past the row's end in its last iteration: nothing to
+// any sum, its exponent finite and far below that of any reference in base 2.
+constexpr float PAD = -1.0e38f;
 
 template <class D>
 struct RowChunk;
@@ -92,16 +101,37 @@ struct Acc {
 // fma(x, log2(e), -mb) with mb = RN(m log2(e)), so that is mb / log2(e) and
 // not m: half an ulp of mb is up to 3e-7 of every term of the thread.  (255
 // f32 rows of V = 50257 with KL, from 64 bits: 3.5e-7 with m, 3.2e-7 with
-// mb / log2(e); entropies of scores around 12: 6.4e-8 and 2.6e-8.)  Where mb overflows (a mask of the type's lowest value) the
-// exponents are (x - m) log2(e).
-__device__ __forceinline__ bool base2_ok(float m) { return __builtin_fabsf(m * LOG2E_F) != __builtin_inff(); }
+// mb / log2(e); entropies of scores around 12: 6.4e-8 and 2.6e-8.)  From 2^31 on
+// (a mask value as a thread's reference) that half ulp, 2^6 and more, would
+// leave the float range as an exponent: the exponents are (x - m) log2(e) there.
+__device__ __forceinline__ bool base2_ok(float m) { return __builtin_fabsf(m * LOG2E_F) < 0x1p31f; }
 __device__ __forceinline__ double ref_of(float m) {
+#pragma clang fp contract(off)
   return base2_ok(m) ? static_cast<double>(m * LOG2E_F) * INV_LOG2E_F : static_cast<double>(m);
+}
+
+// (Products and sums are fused where written as fma only, here and in the
+// kernel: the same bits from every instantiation.)
+// One value below the reference m: its base-2 exponent, and whether that is
+// -inf though the value is finite (the difference is past the float range).
+struct Below {
+  float d2;
+  bool under;
+  // the base-2 difference itself
+  __device__ __forceinline__ double wide(float x, float m) const {
+    return under ? (static_cast<double>(x) - ref_of(m)) * static_cast<double>(LOG2E_F) : static_cast<double>(d2);
+  }
+};
+__device__ __forceinline__ Below below(float x, float m) {
+  if (x == -__builtin_inff()) return {x, false};
+  const float d2 = base2_ok(m) ? fmaf(x, LOG2E_F, -(m * LOG2E_F)) : (x - m) * LOG2E_F;
+  return {d2, d2 == -__builtin_inff()};
 }
 
 // Re-base a partial on a larger maximum M (m <= M).  A partial with no
 // element yet (m == -inf) has zero sums and stays zero.
 __device__ __forceinline__ void rebase_x(Acc& a, float M) {
+#pragma clang fp contract(off)
   if (a.m == M || a.m == -__builtin_inff()) {
     a.m = M;
     return;
@@ -114,6 +144,7 @@ __device__ __forceinline__ void rebase_x(Acc& a, float M) {
   a.m = M;
 }
 __device__ __forceinline__ void rebase_y(Acc& a, float M) {
+#pragma clang fp contract(off)
   if (a.my == M || a.my == -__builtin_inff()) {
     a.my = M;
     return;
@@ -127,18 +158,39 @@ __device__ __forceinline__ void rebase_y(Acc& a, float M) {
 
 }  // namespace
 
-template <class D, bool KL, int NT_RS>
-__global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) {
+// A row's terms are grouped by its length and type alone, so that a row has the
+// same bits in any call: 256 lanes take the row's iterations (RS_U chunks per
+// lane) in up to RS_SEGS runs, a lane's terms of one run go into one partial,
+// and the partials merge wave by wave, then run by run.  How many of the runs
+// are taken side by side, by 256 threads each, is the launch's choice.
+constexpr int RS_LANES = 256;
+constexpr int RS_WAVES = RS_LANES / WAVE;
+constexpr int RS_U = 2;     // chunks per lane in flight
+constexpr int RS_SEGS = 4;  // most runs of a row
+
+// Runs of a row of `iters` iterations, a power of two, each of four iterations
+// or more: of two, the merges cost many rows more than the split gives few (4096
+// bf16 rows of V = 32000 with KL: 90 us in two runs, 100 in four; 255 rows 12.4
+// and 11.8).
+__host__ __device__ __forceinline__ int rs_segs(int iters) { return iters >= 4 * RS_SEGS ? RS_SEGS : iters >= 8 ? 2 : 1; }
+template <class D>
+__host__ __device__ __forceinline__ int rs_iters(int V) {
+  constexpr int E = RS_LANES * RS_U * RowChunk<D>::N;
+  return (V + E - 1) / E;
+}
+
+// GROUPS: runs taken side by side (a divisor of the row's number of runs)
+template <class D, bool KL, int GROUPS>
+__global__ __launch_bounds__(RS_LANES * GROUPS) void k_row_stats(const fl_row_stats_args a) {
+#pragma clang fp contract(off)
   using C = RowChunk<D>;
   constexpr int N = C::N;
-  constexpr int NW_RS = NT_RS / WAVE;
-  // chunks per thread in flight: with 4 the 16-bit instantiations hold too
-  // many registers for the waves that keep HBM busy (4096 bf16 rows of V =
-  // 128256: 188 us at 4, 174 us at 2, 6.0 TB/s; with KL, 2048 rows: 218 / 214 us)
-  constexpr int U_RS = 2;
-  __shared__ Acc part[NW_RS];
-  __shared__ float ref_m[NW_RS], ref_my[NW_RS];
-  const int tid = threadIdx.x;
+  constexpr int NPART = RS_SEGS * RS_WAVES;
+  static_assert(NPART <= WAVE, "one lane per partial");
+  __shared__ Acc part[NPART];
+  __shared__ float ref_m[RS_WAVES], ref_my[RS_WAVES];
+  const int tid = threadIdx.x, lane = tid & (WAVE - 1);
+  const int slot = tid % RS_LANES;  // the thread's lane of its run
   const int64_t r = blockIdx.x;
   const int V = static_cast<int>(a.vocab);
   const size_t esz = D::id == FL_DTYPE_F32 ? 4 : 2;
@@ -146,55 +198,82 @@ __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) 
   const char* yp = KL ? static_cast<const char*>(a.ref_logits) + r * a.ref_ld * esz : xp;
   const __amdgpu_buffer_rsrc_t rx = row_rsrc(xp, static_cast<uint32_t>(V * esz));
   const __amdgpu_buffer_rsrc_t ry = row_rsrc(yp, static_cast<uint32_t>(V * esz));
-  const int nch = (V + N - 1) / N;
   const int nfull = V / N;
+  const int iters = rs_iters<D>(V), nseg = rs_segs(iters), per = (iters + nseg - 1) / nseg;
 
-  Acc acc = {-__builtin_inff(), 0.0, 0.0, -__builtin_inff(), 0.0, 0.0};
-  auto load = [&](__amdgpu_buffer_rsrc_t rs, int c, float (&x)[N]) __attribute__((always_inline)) {
-    if (c < nfull) {
-      C::unpack(buf_load16_once(rs, 16u * c, 0u), x);  // (read once: 207 -> 201 us at 4096 x 128256 bf16)
-    } else {
+  // (the sum is not asked for, or the wave has seen a -inf logit and it is NaN)
+  bool lost_u = a.out_entropy == nullptr, lost_w = a.out_kl == nullptr;
+  for (int seg = __builtin_amdgcn_readfirstlane(tid / RS_LANES); seg < nseg; seg += GROUPS) {
+    Acc acc = {-__builtin_inff(), 0.0, 0.0, -__builtin_inff(), 0.0, 0.0};
+    for (int it = seg * per; it < min(iters, (seg + 1) * per); ++it) {
+      const int base = it * RS_U * RS_LANES, c0 = base + slot;
+      // (chunks past the row, and what lies past it of the last one, load zeros:
+      // the range check goes by dwords)
+      uint4 qx[RS_U], qy[RS_U];
 #pragma unroll
-      for (int e = 0; e < N; ++e) x[e] = N * c + e < V ? C::elem(rs, N * c + e) : -__builtin_inff();
-    }
-  };
-  for (int c0 = 0; c0 < nch; c0 += U_RS * NT_RS) {
-    float xs[U_RS][N], ys[U_RS][N];
-#pragma unroll
-    for (int k = 0; k < U_RS; ++k) {
-      const int c = c0 + k * NT_RS + tid;
-      if (c < nch) {
-        load(rx, c, xs[k]);
-        if (KL) load(ry, c, ys[k]);
-      } else {
-#pragma unroll
-        for (int e = 0; e < N; ++e) xs[k][e] = ys[k][e] = -__builtin_inff();
+      for (int k = 0; k < RS_U; ++k) {
+        // (read once: 207 -> 201 us at 4096 x 128256 bf16)
+        qx[k] = buf_load16_once(rx, 16u * static_cast<uint32_t>(c0 + k * RS_LANES), 0u);
+        if (KL) qy[k] = buf_load16_once(ry, 16u * static_cast<uint32_t>(c0 + k * RS_LANES), 0u);
       }
-    }
-    // maxima of the iteration's chunks first (padding is -inf)
-    float cm = xs[0][0], cmy = ys[0][0];
+      float xs[RS_U][N], ys[RS_U][N];
 #pragma unroll
-    for (int k = 0; k < U_RS; ++k)
-#pragma unroll
-      for (int e = 0; e < N; ++e) {
-        cm = fmaxf(cm, xs[k][e]);
-        if (KL) cmy = fmaxf(cmy, ys[k][e]);
+      for (int k = 0; k < RS_U; ++k) {
+        C::unpack(qx[k], xs[k]);
+        if (KL) C::unpack(qy[k], ys[k]);
       }
-    if (cm > acc.m + SLACK) rebase_x(acc, cm);
-    if (KL && cmy > acc.my + SLACK) rebase_y(acc, cmy);
-    // exponents in base 2: d2 = (x - m) log2(e) in one rounding; the base-2
-    // sums of the iteration (at most U_RS * N terms, each below e^SLACK) are
-    // scaled to natural units and added to the float64 partials once
-    const float mb = acc.m * LOG2E_F, myb = acc.my * LOG2E_F;
-    float fs = 0.0f, fu = 0.0f, fsy = 0.0f, fw = 0.0f;
-    double wd = 0.0;
-    const bool bx = base2_ok(acc.m), by = !KL || base2_ok(acc.my);
-    bool general = !(c0 + (U_RS - 1) * NT_RS + tid < nfull && bx && by);
-    if (!general) {
-      // whole chunks under a finite maximum: -inf gives d2 = -inf, e = 0 and
-      // e * d2 = NaN, the reference's 0 * -inf
+      const bool whole = base + RS_U * RS_LANES <= nfull;  // (for all lanes)
+      if (!whole) {
+        // past the row -inf (for the maximum); the last value of an odd 16-bit
+        // row, whose dword reaches past it, by itself
+        if (N * c0 >= V) continue;
 #pragma unroll
-      for (int k = 0; k < U_RS; ++k)
+        for (int k = 0; k < RS_U; ++k)
+#pragma unroll
+          for (int e = 0; e < N; ++e) {
+            const int i = N * (c0 + k * RS_LANES) + e;
+            if (i >= V) {
+              xs[k][e] = -__builtin_inff();
+              if (KL) ys[k][e] = -__builtin_inff();
+            } else if (D::id != FL_DTYPE_F32 && e % 2 == 0 && i == V - 1) {
+              xs[k][e] = C::elem(rx, i);
+              if (KL) ys[k][e] = C::elem(ry, i);
+            }
+          }
+      }
+      // maxima of the iteration's chunks first (padding is -inf)
+      float cm = xs[0][0], cmy = ys[0][0];
+#pragma unroll
+      for (int k = 0; k < RS_U; ++k)
+#pragma unroll
+        for (int e = 0; e < N; ++e) {
+          cm = fmaxf(cm, xs[k][e]);
+          if (KL) cmy = fmaxf(cmy, ys[k][e]);
+        }
+      if (cm > acc.m + SLACK) rebase_x(acc, cm);
+      if (KL && cmy > acc.my + SLACK) rebase_y(acc, cmy);
+      // exponents in base 2: d2 = (x - m) log2(e) in one rounding; the base-2
+      // sums of the iteration (at most RS_U * N terms, each below e^SLACK) are
+      // scaled to natural units and added to the float64 partials once
+      // (without a reference, -inf values alone so far, relative to 0: their
+      // terms are the same)
+      const float mb = acc.m == -__builtin_inff() ? 0.0f : acc.m * LOG2E_F;
+      const float myb = acc.my == -__builtin_inff() ? 0.0f : acc.my * LOG2E_F;
+      float fs = 0.0f, fu = 0.0f, fsy = 0.0f, fw = 0.0f;
+      if (!whole) {
+        // (then a finite value whose terms are 0)
+#pragma unroll
+        for (int k = 0; k < RS_U; ++k)
+#pragma unroll
+          for (int e = 0; e < N; ++e)
+            if (N * (c0 + k * RS_LANES) + e >= V) {
+              xs[k][e] = PAD;
+              if (KL) ys[k][e] = PAD;
+            }
+      }
+      // -inf gives d2 = -inf, e = 0 and e * d2 = NaN, the reference's 0 * -inf
+#pragma unroll
+      for (int k = 0; k < RS_U; ++k)
 #pragma unroll
         for (int e = 0; e < N; ++e) {
           const float d2 = fmaf(xs[k][e], LOG2E_F, -mb);
@@ -207,107 +286,134 @@ __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) 
             fw = fmaf(ex, d2 - dy2, fw);
           }
         }
-    }
-    // A finite value near the type's lowest (a mask) has d2 = -inf too, where
-    // the reference's 0 * x is 0 (and p * -y large, but finite): such an
-    // iteration is taken again below.  Not once a -inf logit has made the
-    // wave's sum NaN, and the row's with it, so that a row with many of them
-    // takes one such iteration a wave.
-    const bool nan_u = !(__builtin_fabsf(fu) < __builtin_inff());
-    const bool nan_w = KL && !(__builtin_fabsf(fw) < __builtin_inff());
-    if (__any(nan_u || nan_w)) {
-      const bool lost_u = __any(acc.u != acc.u), lost_w = KL && __any(acc.w != acc.w);
-      general = general || (nan_u && !lost_u) || (nan_w && !lost_w);
-    }
-    if (general) {
-      // the row's last chunks (partial or past the row), values before any
-      // finite one (-inf below a maximum that is still -inf), references whose
-      // base-2 form overflows, and values whose exponent does
-      auto below = [](float x, float m, float b, bool ok) {
-        return x == -__builtin_inff() ? x : ok ? fmaf(x, LOG2E_F, -b) : (x - m) * LOG2E_F;
-      };
-      // (the difference itself, also where it is past the float range)
-      auto wide = [](float d2, float x, float m) -> double {
-        return d2 == -__builtin_inff() && x != d2 ? (static_cast<double>(x) - ref_of(m)) * LOG2E_F : d2;
-      };
-      fs = fu = fsy = 0.0f;
-      fw = 0.0f;
+      // A finite value near the type's lowest (a mask) has d2 = -inf too, where
+      // the reference's 0 * x is 0 (and p * -y large, but finite); and a thread's
+      // reference may be such a value.  Such an iteration is taken again, from
+      // memory and in float64 where float ends.  Not once a -inf logit has
+      // made the wave's sum NaN, and the row's with it, so that a row with many
+      // of them takes one such iteration a wave.
+      const bool off = !(__builtin_fabsf(mb) < 0x1p31f) || (KL && !(__builtin_fabsf(myb) < 0x1p31f));
+      const bool nan_u = !(__builtin_fabsf(fu) < __builtin_inff());
+      const bool nan_w = KL && !(__builtin_fabsf(fw) < __builtin_inff());
+      double wd = 0.0;
+      if (__any(off || nan_u || nan_w)) {
+        lost_u = lost_u || __any(acc.u != acc.u);
+        lost_w = lost_w || (KL && __any(acc.w != acc.w));
+        if (off || (nan_u && !lost_u) || (nan_w && !lost_w)) {
+          fs = fu = fsy = fw = 0.0f;
+#pragma unroll 1
+          for (int k = 0; k < RS_U; ++k) {
+            const int c = c0 + k * RS_LANES;
+            float x[N], y[N];
+            C::unpack(buf_load16(rx, 16u * static_cast<uint32_t>(c), 0u), x);
+            if (KL) C::unpack(buf_load16(ry, 16u * static_cast<uint32_t>(c), 0u), y);
 #pragma unroll
-      for (int k = 0; k < U_RS; ++k) {
-        const int c = c0 + k * NT_RS + tid;
-#pragma unroll
-        for (int e = 0; e < N; ++e) {
-          if (N * c + e >= V) continue;
-          const float x = xs[k][e], d2 = below(x, acc.m, mb, bx);
-          const float ex = __builtin_amdgcn_exp2f(d2);
-          fs += ex;
-          fu += d2 == -__builtin_inff() && x != d2 ? 0.0f : ex * d2;
-          if (KL) {
-            const float y = ys[k][e], dy2 = below(y, acc.my, myb, by);
-            fsy += __builtin_amdgcn_exp2f(dy2);
-            wd += static_cast<double>(ex) * (wide(d2, x, acc.m) - wide(dy2, y, acc.my));
+            for (int e = 0; e < N; ++e) {
+              const int i = N * c + e;
+              if (i >= V) continue;
+              if (D::id != FL_DTYPE_F32 && e % 2 == 0 && i == V - 1) {
+                x[e] = C::elem(rx, i);
+                if (KL) y[e] = C::elem(ry, i);
+              }
+              const Below bx = below(x[e], acc.m);
+              const float ex = __builtin_amdgcn_exp2f(bx.d2);
+              fs += ex;
+              fu += bx.under ? 0.0f : ex * bx.d2;
+              if (KL) {
+                const Below by = below(y[e], acc.my);
+                fsy += __builtin_amdgcn_exp2f(by.d2);
+                wd += static_cast<double>(ex) * (bx.wide(x[e], acc.m) - by.wide(y[e], acc.my));
+              }
+            }
           }
         }
       }
+      acc.s += fs;
+      acc.u = fma(static_cast<double>(fu), INV_LOG2E_F, acc.u);
+      if (KL) {
+        acc.sy += fsy;
+        acc.w = fma(static_cast<double>(fw) + wd, INV_LOG2E_F, acc.w);
+      }
     }
-    acc.s += fs;
-    acc.u += static_cast<double>(fu) * INV_LOG2E_F;
-    if (KL) {
-      acc.sy += fsy;
-      acc.w += (static_cast<double>(fw) + wd) * INV_LOG2E_F;
-    }
-  }
-  // merge: the row's largest references first, so that each thread re-bases
-  // its partial once (two double-precision exponentials), then plain sums in a
-  // fixed tree.  (Merging partial by partial re-based twice per step of the
-  // tree: 4096 bf16 rows of V = 4099 took 38.0 us, now 28.6.)
-  const int wave = tid / WAVE;
-  const float wm = wave_reduce(acc.m, OpMax()), wmy = KL ? wave_reduce(acc.my, OpMax()) : 0.0f;
-  if ((tid & (WAVE - 1)) == 0) {
-    ref_m[wave] = wm;
-    ref_my[wave] = wmy;
-  }
-  __syncthreads();
-  float M = ref_m[0], My = ref_my[0];
+    // the wave's partial: its largest references first (of a row of one run, the
+    // row's), so that each lane re-bases its own once, then plain sums in a
+    // fixed tree.  (Merging partial by partial re-based twice per step of the
+    // tree: 4096 bf16 rows of V = 4099 took 38.0 us, now 15.6.)
+    const int wave = slot / WAVE;
+    float M = wave_reduce(acc.m, OpMax()), My = KL ? wave_reduce(acc.my, OpMax()) : 0.0f;
+    if (nseg == 1) {  // (every wave of the group is here)
+      if (lane == 0) {
+        ref_m[wave] = M;
+        ref_my[wave] = My;
+      }
+      __syncthreads();
 #pragma unroll
-  for (int i = 1; i < NW_RS; ++i) {
-    M = fmaxf(M, ref_m[i]);
-    My = fmaxf(My, ref_my[i]);
-  }
-  rebase_x(acc, M);
-  if (KL) rebase_y(acc, My);  // (from the thread's own s: before the sums)
-  acc.s = wave_reduce(acc.s, OpAdd());
-  acc.u = wave_reduce(acc.u, OpAdd());
-  if (KL) {
-    acc.sy = wave_reduce(acc.sy, OpAdd());
-    acc.w = wave_reduce(acc.w, OpAdd());
-  }
-  // (field by field: a copy of the struct keeps it in memory, which the compiler
-  // puts into LDS, indexed through the launch packet in host memory: 255 bf16
-  // rows of V = 512 18.2 us, now 4.7)
-  if ((tid & (WAVE - 1)) == 0) {
-    Acc& p = part[wave];
-    p.m = acc.m;
-    p.s = acc.s;
-    p.u = acc.u;
+      for (int i = 0; i < RS_WAVES; ++i) {
+        M = fmaxf(M, ref_m[i]);
+        My = fmaxf(My, ref_my[i]);
+      }
+    }
+    rebase_x(acc, M);
+    if (KL) rebase_y(acc, My);  // (from the lane's own s: before the sums)
+    acc.s = wave_reduce(acc.s, OpAdd());
+    acc.u = wave_reduce(acc.u, OpAdd());
     if (KL) {
-      p.my = acc.my;
-      p.sy = acc.sy;
-      p.w = acc.w;
+      acc.sy = wave_reduce(acc.sy, OpAdd());
+      acc.w = wave_reduce(acc.w, OpAdd());
+    }
+    // (field by field: a copy of the struct keeps it in memory, which the
+    // compiler puts into LDS, indexed through the launch packet in host memory:
+    // 12 us of every launch: 255 bf16 rows of V = 512 18.2 us so, 4.1 without)
+    if (lane == 0) {
+      Acc& p = part[seg * RS_WAVES + wave];
+      p.m = acc.m;
+      p.s = acc.s;
+      p.u = acc.u;
+      if (KL) {
+        p.my = acc.my;
+        p.sy = acc.sy;
+        p.w = acc.w;
+      }
     }
   }
   __syncthreads();
+  if (tid >= NPART) return;
+  Acc t = {-__builtin_inff(), 0.0, 0.0, -__builtin_inff(), 0.0, 0.0};
+  if (nseg == 1) {
+    // the waves' partials, relative to the row's references, in order
+    t.m = part[0].m;
+    if (KL) t.my = part[0].my;
+#pragma unroll
+    for (int i = 0; i < RS_WAVES; ++i) {
+      t.s += part[i].s;
+      t.u += part[i].u;
+      if (KL) {
+        t.sy += part[i].sy;
+        t.w += part[i].w;
+      }
+    }
+  } else {
+    // lane i takes partial i: as above, and again a fixed tree
+    if (tid < nseg * RS_WAVES) {
+      t.m = part[tid].m;
+      t.s = part[tid].s;
+      t.u = part[tid].u;
+      if (KL) {
+        t.my = part[tid].my;
+        t.sy = part[tid].sy;
+        t.w = part[tid].w;
+      }
+    }
+    rebase_x(t, wave_reduce<float, OpMax, NPART>(t.m, OpMax()));
+    if (KL) rebase_y(t, wave_reduce<float, OpMax, NPART>(t.my, OpMax()));
+    t.s = wave_reduce<double, OpAdd, NPART>(t.s, OpAdd());
+    t.u = wave_reduce<double, OpAdd, NPART>(t.u, OpAdd());
+    if (KL) {
+      t.sy = wave_reduce<double, OpAdd, NPART>(t.sy, OpAdd());
+      t.w = wave_reduce<double, OpAdd, NPART>(t.w, OpAdd());
+    }
+  }
   if (tid != 0) return;
-  Acc t = {M, 0.0, 0.0, My, 0.0, 0.0};
-#pragma unroll
-  for (int i = 0; i < NW_RS; ++i) {
-    t.s += part[i].s;
-    t.u += part[i].u;
-    if (KL) {
-      t.sy += part[i].sy;
-      t.w += part[i].w;
-    }
-  }
   const double logS = log(t.s);
   if (a.out_entropy) a.out_entropy[r] = static_cast<float>(logS - t.u / t.s);
   if (a.out_lse) a.out_lse[r] = static_cast<float>(ref_of(t.m) + logS);
@@ -322,24 +428,36 @@ __global__ __launch_bounds__(NT_RS) void k_row_stats(const fl_row_stats_args a) 
   }
 }
 
-// Threads per row: 256 where rows are many (their merges overlap other rows'
-// reads); 1024 where a CU gets one row at most, so that the row has 16 waves'
-// loads in flight instead of 4.  f32 with KL, V = 50257: 255 rows 34.2 us with
-// 256 threads, 22.2 us with 1024; 520 rows 41.4 against 47.9 us.
-constexpr int64_t RS_FEW_ROWS = 256;
+// Runs taken side by side (as far as the row has so many): four, unless the
+// launch has rows enough for the CUs and the KL's registers would leave a CU one
+// or two work-groups of that size.  Per launch with four / two / one: f32 V =
+// 50257 255 rows 12.0 / 16.4 / 25.2 us, 512 20.9 / 20.7 / 28.2, 2048 65.5 / 69.0 /
+// 72.2; bf16 4096x128256 175 / 178 / 178; f32 with KL V = 32000 255 rows 18.4 /
+// 18.7 / 25.5, 257 23.5 / 22.0 / 27.1, 1024 53.2 / 48.7 / 48.4, 4096 178 / 164 /
+// 166; bf16 with KL V = 32000 (two runs) 512 rows - / 19.3 / 21.4, 4096 - / 109 / 99.
+constexpr int64_t RS_CU_ROWS = 256, RS_MANY_ROWS = 1024;
+int rs_groups(bool kl, bool f32, int64_t rows) {
+  if (!kl || rows <= RS_CU_ROWS) return 4;
+  return f32 || rows <= RS_MANY_ROWS ? 2 : 1;
+}
 
 hipError_t launch_row_stats(const fl_row_stats_args& a, hipStream_t s) {
   const dim3 grid(static_cast<unsigned>(a.rows));
-  const bool few = a.rows <= RS_FEW_ROWS;
   auto run = [&](auto d) {
     using D = decltype(d);
-    auto go = [&](auto kl_c) {
-      constexpr bool KL = decltype(kl_c)::value;
-      if (few) hipLaunchKernelGGL((k_row_stats<D, KL, 1024>), grid, dim3(1024), 0, s, a);
-      else hipLaunchKernelGGL((k_row_stats<D, KL, 256>), grid, dim3(256), 0, s, a);
+    auto go = [&](auto kl_c, auto groups_c) {
+      constexpr int G = decltype(groups_c)::value;
+      hipLaunchKernelGGL((k_row_stats<D, decltype(kl_c)::value, G>), grid, dim3(RS_LANES * G), 0, s, a);
     };
-    if (a.ref_logits != nullptr) go(std::true_type{});
-    else go(std::false_type{});
+    auto go_kl = [&](auto kl_c) {
+      const int nseg = rs_segs(rs_iters<D>(static_cast<int>(a.vocab)));
+      const int groups = std::min(nseg, rs_groups(a.ref_logits != nullptr, a.dtype == FL_DTYPE_F32, a.rows));
+      if (groups == 4) go(kl_c, std::integral_constant<int, 4>{});
+      else if (groups == 2) go(kl_c, std::integral_constant<int, 2>{});
+      else go(kl_c, std::integral_constant<int, 1>{});
+    };
+    if (a.ref_logits != nullptr) go_kl(std::true_type{});
+    else go_kl(std::false_type{});
   };
   if (a.dtype == FL_DTYPE_F32) run(F32{});
   else if (a.dtype == FL_DTYPE_BF16) run(BF16{});

@@ -68,3 +68,22 @@ def test_infinite_masks_beside_finite_ones(dt, R):
     assert bool(torch.isnan(out.entropy[:2]).all()) and bool(torch.isnan(out.kl[:2]).all())
     assert bool(torch.isnan(h[:2]).all()) and float(kl[2]) == float("inf") == float(out.kl[2])
     assert _close(out.entropy[2:], h[2:], 2e-6, 1.0) and _close(out.kl[3:], kl[3:], 2e-6, 2.0)
+
+
+@pytest.mark.parametrize("low", [-3.0e38, -1.7e38, -1.0e38, -6.0e37, -1.0e15, -1.7e9, -1.3e9, -1.0e9])
+@pytest.mark.parametrize("V", [5, 2050, 40003])
+def test_masks_of_any_depth(low, V):
+    """Rows of a mask value alone but for their last, with the row's end inside
+    an iteration: the mask is some lanes' reference."""
+    print(f"[rowstats masks low={low} V={V}]", flush=True)
+    R = 3
+    g = torch.Generator(device="cuda").manual_seed(V)
+    x = torch.full((R, V), low, device="cuda")
+    y = torch.full((R, V), low, device="cuda")
+    x[1:, V - 3:], y[2:, V - 4:] = torch.randn(R - 1, 3, generator=g, device="cuda"), torch.randn(R - 2, 4, generator=g, device="cuda")
+    lab = torch.full((R,), V - 2, device="cuda")
+    out = row_stats(x, lab, y, entropy=True, lse=True)
+    h, kl = _want(x, y)
+    assert _close(out.entropy, h, 2e-6, 1.0) and _close(out.logprob, torch.log_softmax(x.double(), -1)[:, V - 2], 2e-6, 1.0)
+    assert _close(out.lse, torch.logsumexp(x.double(), -1), 2e-6, 1.0)
+    assert _close(out.kl, kl, 2e-6, 2.0), (out.kl, kl)

@@ -20,7 +20,7 @@ def test_no_private_memory_in_lds(tmp_path):
     src, out = os.path.join(B.CSRC, "fl_rowstats.hip"), str(tmp_path / "rs.s")
     subprocess.run([hipcc, *B.HIPCC_FLAGS, "--offload-device-only", "-S", src, "-o", out], check=True, capture_output=True)
     text = open(out).read()
-    assert len(re.findall(r"^\s*\.amdhsa_kernel ", text, flags=re.M)) == 12   # 3 dtypes, with and without KL, 2 work-group sizes
+    assert len(re.findall(r"^\s*\.amdhsa_kernel ", text, flags=re.M)) == 18   # 3 dtypes, with and without KL, 3 splits
     assert set(re.findall(r"\.amdhsa_user_sgpr_dispatch_ptr (\d)", text)) == {"0"}
     assert set(re.findall(r"\.amdhsa_private_segment_fixed_size (\d+)", text)) == {"0"}
     assert max(map(int, re.findall(r"\.amdhsa_group_segment_fixed_size (\d+)", text))) <= 1024
