@@ -40,7 +40,7 @@
 extern "C" {
 #endif
 
-#define FL_ABI_VERSION 5
+#define FL_ABI_VERSION 6
 
 enum fl_dtype { FL_DTYPE_F32 = 0, FL_DTYPE_BF16 = 1, FL_DTYPE_F16 = 2 };
 

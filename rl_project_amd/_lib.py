@@ -18,7 +18,7 @@ import torch  # noqa: F401  (loads the HIP runtime the library binds to)
 LIB_PATH = os.environ.get("FL_SAMPLER_LIB") or os.path.join(os.path.dirname(os.path.abspath(__file__)), "_lib",
                                                             "libflsampler.so")
 
-FL_ABI_VERSION = 5
+FL_ABI_VERSION = 6
 FL_DTYPE_F32, FL_DTYPE_BF16, FL_DTYPE_F16 = 0, 1, 2
 FL_OK, FL_EIO, FL_EINVAL, FL_ENOTSUP = 0, -5, -22, -95
 FL_ROW_OK, FL_ROW_NAN, FL_ROW_INF, FL_ROW_BAD_HISTORY, FL_ROW_LIMIT, FL_ROW_ALL_MASKED = 0, 1, 2, 4, 8, 16
@@ -126,7 +126,15 @@ def lib() -> ctypes.CDLL:
         handle = ctypes.CDLL(LIB_PATH)
     except OSError as exc:  # pragma: no cover - depends on the machine
         raise SamplerLibraryError(f"cannot load {LIB_PATH}: {exc}") from exc
-    handle.fl_abi_version.restype = ctypes.c_int
+    # (before any other symbol is bound: an older library may lack some)
+    try:
+        handle.fl_abi_version.restype = ctypes.c_int
+        version = handle.fl_abi_version()
+    except AttributeError:
+        raise SamplerLibraryError(f"{LIB_PATH} has no fl_abi_version: not this library") from None
+    if version != FL_ABI_VERSION:
+        raise SamplerLibraryError(f"ABI version {version} of {LIB_PATH} != {FL_ABI_VERSION}: "
+                                  "build it with `python -m rl_project_amd.build`")
     handle.fl_last_error.restype = ctypes.c_char_p
     handle.fl_sample.argtypes = [ctypes.POINTER(SampleArgs), _p]
     handle.fl_sample.restype = ctypes.c_int
@@ -150,8 +158,6 @@ def lib() -> ctypes.CDLL:
     handle.fl_lm_head_workspace_bytes.restype = ctypes.c_int
     handle.fl_row_stats.argtypes = [ctypes.POINTER(RowStatsArgs), _p]
     handle.fl_row_stats.restype = ctypes.c_int
-    if handle.fl_abi_version() != FL_ABI_VERSION:
-        raise SamplerLibraryError(f"ABI version {handle.fl_abi_version()} != {FL_ABI_VERSION}")
     _lib = handle
     return handle
 

@@ -299,3 +299,19 @@ def test_lm_head_argument_errors():
         assert needle in L.fl_last_error().decode(), (change, L.fl_last_error())
     a.batch = 0
     assert L.fl_lm_head_sample(ctypes.byref(a), None) == _lib.FL_OK
+
+
+@pytest.mark.parametrize("body", ["int fl_abi_version(void) { return 5; }", "int other(void) { return 0; }"])
+def test_another_version_is_refused_before_its_symbols_are_bound(body, tmp_path, monkeypatch):
+    """A library of another ABI version, or none, is named as such: it may lack
+    the symbols that this version binds."""
+    gcc = shutil.which("gcc")
+    if gcc is None:
+        pytest.skip("gcc not available")
+    (tmp_path / "old.c").write_text(body)
+    path = str(tmp_path / "libold.so")
+    subprocess.run([gcc, "-shared", "-fPIC", str(tmp_path / "old.c"), "-o", path], check=True)
+    monkeypatch.setattr(_lib, "LIB_PATH", path)
+    monkeypatch.setattr(_lib, "_lib", None)
+    with pytest.raises(_lib.SamplerLibraryError, match="version"):
+        _lib.lib()
