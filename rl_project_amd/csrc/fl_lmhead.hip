@@ -103,7 +103,7 @@ struct LmWs {
   uint32_t* cnt;    // [batch, LM_CNT_LD] candidates appended (word 0 of a row's 256 bytes)
   uint32_t* stat;   // [batch] FL_ROW_* bits found by prep and gemm
   uint32_t* bits;   // [batch, bw] history bitmap
-  uint16_t* skey;   // [batch, nsl] bf16 patterns of the sampled logits (entry e: vocabulary row e·S)
+  uint16_t* slogit; // [batch, nsl] bf16 patterns of the sampled logits (entry e: vocabulary row e·S)
   uint64_t* cand;   // [batch, LM_CAP] (key << 32) | ~vocabulary index
   int bw;           // words per bitmap row, a multiple of 4
   int stride;       // S
@@ -144,7 +144,7 @@ inline LmWs lm_ws(void* p, int64_t batch, int64_t vocab) {
   off += lm_align(4 * B);
   w.bits = reinterpret_cast<uint32_t*>(q + off);
   off += lm_align(4 * B * w.bw);
-  w.skey = reinterpret_cast<uint16_t*>(q + off);
+  w.slogit = reinterpret_cast<uint16_t*>(q + off);
   off += lm_align(2 * B * static_cast<size_t>(w.nsl));
   w.cand = reinterpret_cast<uint64_t*>(q + off);
   return w;
@@ -254,7 +254,7 @@ __device__ void lm_prep_row(const fl_lm_head_args& a, const LmWs& ws, int b, uin
 // ---------------------------------------------------------------- sample gemm
 // The sampled rows: vocabulary rows e·S for tile entries e, 16 per wave and 64
 // per work-group (ns / 64 work-groups), their logits' bf16 patterns stored to
-// ws.skey (the thresh kernel transforms them).  Work-groups past those prepare
+// ws.slogit (the thresh kernel transforms them).  Work-groups past those prepare
 // the rows' histories.  MB: 16-row blocks of the batch (1, 2 or 4).  Each
 // 16 x 16 block of logits is one wave's MFMA chain over the dim in 32-wide
 // steps in ascending order, as in the main gemm below, so a sampled value
@@ -362,7 +362,7 @@ __global__ __launch_bounds__(LM_NT) void k_lm_sample(const fl_lm_head_args a, Lm
 #pragma unroll
     for (int r = 0; r < 4; ++r) {
       const int m = 16 * mb + 4 * l4 + r;
-      if (m < B && eme < ns) ws.skey[static_cast<size_t>(m) * ws.nsl + eme] = static_cast<uint16_t>(BF16::from_f32(acc[mb][0][r]));
+      if (m < B && eme < ns) ws.slogit[static_cast<size_t>(m) * ws.nsl + eme] = static_cast<uint16_t>(BF16::from_f32(acc[mb][0][r]));
     }
   }
 }
@@ -657,7 +657,7 @@ __global__ __launch_bounds__(LM_NTT) void k_lm_thresh(const fl_lm_head_args a, L
     const int ns = ws.ns, nj = ns - 8 * tid;   // keys of this thread (8 or more: 8)
     uint32_t key[8];
     if (nj > 0) {
-      const uint4 q = reinterpret_cast<const uint4*>(ws.skey + static_cast<size_t>(b) * ws.nsl)[tid];
+      const uint4 q = reinterpret_cast<const uint4*>(ws.slogit + static_cast<size_t>(b) * ws.nsl)[tid];
       const uint32_t wd[4] = {q.x, q.y, q.z, q.w};
       const uint32_t* hb = ws.bits + static_cast<size_t>(b) * ws.bw;
       uint32_t hw[8];
