@@ -863,7 +863,9 @@ __device__ __forceinline__ bool row_body(const fl_sample_args a, const int SC_EL
   bool done = false;
   if constexpr (!HEAVY) {
     const bool tk = K > 0 && K < V;
-    const int most = N > NT ? SHORT_MAX : (TP > 0.0f && TP < 1.0f) || MP > 0.0f ? SHORT_CUT : SHORT_PLAIN;
+    // (without short circuits, which would be branches)
+    const bool cuts = ((TP > 0.0f) & (TP < 1.0f)) | (MP > 0.0f);
+    const int most = N > NT ? SHORT_MAX : cuts ? SHORT_CUT : SHORT_PLAIN;
     if (N > 0 && (N <= most || (tk && K <= SHORT_MAX))) {  // block-uniform
       if (tid < WAVE) {
         float* const Ys = reinterpret_cast<float*>(sh.hist + SLICE_BASE);
