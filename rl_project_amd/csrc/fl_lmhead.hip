@@ -622,7 +622,7 @@ __global__ __launch_bounds__(NW * WAVE) __attribute__((amdgpu_waves_per_eu(NW / 
 // and keeps its eight transformed keys in registers for two passes of a
 // histogram in LDS: the upper 12 bits, then the lower 4 within the chosen bin.
 // (With 8 + 8 bits, nearly all of a row's keys fell into some ten bins of the
-// first pass and their atomics queued, 64x4096x128256: 9.8 us, now 9.3 with
+// first pass and their atomics queued.  64x4096x128256: 9.7 us so, 9.8 now with
 // the transforms that the sample gemm did before.)
 // Soft-cap, penalty and temperature are monotone (non-decreasing) in the
 // logit, separately for history members and the rest, so "transformed key

@@ -10,7 +10,9 @@ Drop-ins with the reference's signatures and results (float32, shapes
 * ``kl_full_distribution(new_logits, ref_logits)`` -- ``training/common/logprobs.py:58-62``
 
 ``row_stats`` returns any combination of them (plus log-sum-exp) from one
-read of the logits.  Logits must be on the ROCm device; there is no CPU path.
+read of the logits.  A row's results are a function of the row alone: the same
+bits in a call of any number of rows.  Logits must be on the ROCm device; there
+is no CPU path.
 """
 
 from __future__ import annotations

@@ -25,8 +25,8 @@ def _check(x, y, lab, tol, per_row=None):
         assert torch.allclose(got, w, rtol=tol, atol=tol * (1.0 + float(w.abs().max()))), (name, float((got - w).abs().max()))
 
 
-# one row per CU and more (256 / 257 rows: 1024 / 256 threads a row); rows shorter
-# than an iteration, its edges, and several iterations
+# one row per CU and more (256 / 257 rows: a KL's runs go side by side in fours or
+# twos); rows shorter than an iteration, its edges, and several iterations
 @pytest.mark.parametrize("R", [1, 256, 257])
 @pytest.mark.parametrize("V", [1, 7, 2047, 2048, 2049, 4096, 8193, 16385])
 @pytest.mark.parametrize("dt", [torch.float32, torch.bfloat16])
